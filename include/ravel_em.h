@@ -281,6 +281,24 @@ int ravel_em_latest1_linear_fwd(const void* write_addr, const void* read_addr, i
                                 size_t workspace_bytes, void* stream);
 
 /*
+ * Weight gradient of ravel_em_latest1_linear_fwd (grad_weight of
+ * ravel_lm/triton_memory.py:428-475):
+ *   grad_weight[m, c*P + p] = sum_{b,t} grad_out[b,t,m] * values[b,t,c,p]
+ * with values the looked-up rows, gathered through src [B,T,C] (the forward's
+ * out_src) and never stored; fp32 accumulation in a fixed order, rounded once
+ * to the payload dtype.  bf16 / f16 payload, grad_out [B,T,M] and grad_weight
+ * [M, C*P] of one dtype, P % 8 == 0, M % 8 == 0, 16-byte aligned payload and
+ * grad_out (RAVEL_EM_EINVAL otherwise).
+ */
+size_t ravel_em_latest1_linear_bwd_weight_workspace(int64_t B, int64_t T, int64_t C, int64_t P,
+                                                    int64_t M);
+int ravel_em_latest1_linear_bwd_weight(const void* payload, const int32_t* src,
+                                       const void* grad_out, int payload_dtype, int64_t B,
+                                       int64_t T, int64_t C, int64_t P, int64_t M,
+                                       void* grad_weight, void* workspace,
+                                       size_t workspace_bytes, void* stream);
+
+/*
  * Backward of causal_last_k_lookup (autograd of ravel_memory.py:173-175;
  * GPU arm triton_latest1.py:132-142): grad_payload[src] += grad_values.
  * Deterministic (bit-identical across runs) in both forms: `chain` = 1 is the

@@ -1170,6 +1170,40 @@ int ravel_em_gather_rows(const void* rows, int64_t n_src, int64_t row_bytes, con
   return RAVEL_EM_OK;
 }
 
+size_t ravel_em_latest1_linear_bwd_weight_workspace(int64_t B, int64_t T, int64_t C, int64_t P,
+                                                    int64_t M) {
+  if (check_tape(B, T, C, 1) || P < 1 || M < 1 || B * T * C == 0) return 0;
+  int64_t k, mk;
+  if (!mul_ok(C, P, &k) || !mul_ok(M, k, &mk) || mk > ((int64_t)1 << 40)) return 0;
+  return weight_grad_floats(B * T, C, P, M) * sizeof(float);
+}
+
+int ravel_em_latest1_linear_bwd_weight(const void* payload, const int32_t* src,
+                                       const void* grad_out, int payload_dtype, int64_t B,
+                                       int64_t T, int64_t C, int64_t P, int64_t M,
+                                       void* grad_weight, void* workspace,
+                                       size_t workspace_bytes, void* stream) {
+  g_err.clear();
+  if (int rc = check_tape(B, T, C, 1)) return rc;  // int32 sources: N < 2^31
+  if (P < 1 || M < 1) return fail(RAVEL_EM_EINVAL, "P and M must be positive");
+  if (B * T * C == 0) return fail(RAVEL_EM_EINVAL, "the weight gradient needs at least one record");
+  if (!payload || !src || !grad_out || !grad_weight) return fail(RAVEL_EM_EINVAL, "null pointer");
+  if (!weight_grad_apply(payload_dtype, B * T, C, P, M, payload, grad_out, grad_weight))
+    return fail(RAVEL_EM_EINVAL,
+                "the weight gradient takes bf16 or f16, P %% 8 == 0, M %% 8 == 0 and 16-byte "
+                "aligned payload and grad_out (dtype %d P=%lld M=%lld)",
+                payload_dtype, (long long)P, (long long)M);
+  const size_t need = ravel_em_latest1_linear_bwd_weight_workspace(B, T, C, P, M);
+  if (need == 0) return fail(RAVEL_EM_EINVAL, "weight of M=%lld x C*P=%lld is too large",
+                             (long long)M, (long long)(C * P));
+  if (!workspace || workspace_bytes < need)
+    return fail(RAVEL_EM_EWORKSPACE, "workspace of %zu bytes, need %zu", workspace_bytes, need);
+  const hipError_t e = weight_grad(payload, src, grad_out, payload_dtype, B * T, C, P, M,
+                                   (float*)workspace, grad_weight, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "weight gradient");
+  return RAVEL_EM_OK;
+}
+
 size_t ravel_em_latest_k_bwd_workspace(int64_t B, int64_t T, int64_t C, int64_t D, int64_t k,
                                        int payload_dtype, int chain) {
   if (k < 1 || D < 1 || check_tape(B, T, C, 1) || check_rows(B, T, C, 1, k)) return 0;

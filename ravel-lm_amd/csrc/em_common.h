@@ -278,6 +278,14 @@ bool gather_gemm_apply(int dtype, int64_t P, int64_t M, const void* payload, con
                        const void* out);
 hipError_t gather_gemm(const void* payload, const int32_t* src, const void* W, int dtype,
                        int64_t NR, int64_t C, int64_t P, int64_t M, void* out, hipStream_t s);
+// Weight gradient of the same map: gw [M][C*P] = grad [NR][M]^T x looked-up
+// rows; part holds weight_grad_floats() fp32 partial sums.
+bool weight_grad_apply(int dtype, int64_t NR, int64_t C, int64_t P, int64_t M, const void* payload,
+                       const void* grad, const void* gw);
+size_t weight_grad_floats(int64_t NR, int64_t C, int64_t P, int64_t M);
+hipError_t weight_grad(const void* payload, const int32_t* src, const void* grad, int dtype,
+                       int64_t NR, int64_t C, int64_t P, int64_t M, float* part, void* gw,
+                       hipStream_t s);
 // Segment-major sources -> record-major (a no-op layout change when C == 1).
 // k <= kTransposeMaxK (one time step's slots of a head fit the LDS tile).
 constexpr int kTransposeMaxK = 4096;

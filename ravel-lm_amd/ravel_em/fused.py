@@ -71,6 +71,47 @@ def _latest1_linear_fake(write_addresses, payloads, read_addresses, weight, addr
             torch.empty(B, T, C, dtype=torch.int32, device=payloads.device))
 
 
+@torch.library.custom_op("ravel_em::latest1_weight_grad", mutates_args=())
+def _weight_grad(payloads: Tensor, src: Tensor, grad2d: Tensor) -> Tensor:
+    """grad2d^T [M, B*T] times the looked-up rows [B*T, C*P] (zeros where src < 0)."""
+    B, T, C, P = payloads.shape
+    M = grad2d.shape[1]
+    # the kernel's forms: whole 16-byte units of both operands' rows
+    if (payloads.dtype in (torch.bfloat16, torch.float16) and P % 8 == 0 and M % 8 == 0 and M > 0
+            and src.numel() > 0 and payloads.data_ptr() % 16 == 0 and grad2d.data_ptr() % 16 == 0):
+        lib = nat.library()
+        out = payloads.new_empty(M, C * P)
+        ws = nat.workspace(lib.ravel_em_latest1_linear_bwd_weight_workspace(B, T, C, P, M),
+                           payloads.device)
+        nat.check(lib.ravel_em_latest1_linear_bwd_weight(
+            nat.ptr(payloads), nat.ptr(src), nat.ptr(grad2d), nat.payload_code(payloads.dtype),
+            B, T, C, P, M, nat.ptr(out), nat.ptr(ws), ws.numel(), nat.stream_of(payloads)))
+        return out
+    rows = gather_read_rows(payloads, src)
+    return torch.matmul(grad2d.t(), rows.reshape(B * T, C * P))
+
+
+@_weight_grad.register_fake
+def _weight_grad_fake(payloads, src, grad2d):
+    B, T, C, P = payloads.shape
+    return payloads.new_empty(grad2d.shape[1], C * P)
+
+
+def _weight_grad_setup(ctx, inputs, output):
+    ctx.save_for_backward(inputs[0], inputs[1])
+
+
+def _weight_grad_backward(ctx, gg):
+    # linear in grad2d; the sources and payload rows carry no second gradient
+    payloads, src = ctx.saved_tensors
+    B, T, C, P = payloads.shape
+    rows = gather_read_rows(payloads, src).reshape(B * T, C * P)
+    return None, None, torch.matmul(rows, gg.t()) if ctx.needs_input_grad[2] else None
+
+
+_weight_grad.register_autograd(_weight_grad_backward, setup_context=_weight_grad_setup)
+
+
 def _setup(ctx, inputs, output):
     write_addresses, payloads, read_addresses, weight, address_space = inputs
     _, src = output
@@ -88,8 +129,7 @@ def _grads(ctx, grad_out, need_payload: bool, need_weight: bool):
     grad2d = grad_out.reshape(B * T, M).to(payloads.dtype)
     grad_weight = grad_payload = None
     if need_weight:
-        read_flat = gather_read_rows(payloads, src)
-        grad_weight = torch.matmul(grad2d.t(), read_flat.reshape(B * T, C * P)).to(weight.dtype)
+        grad_weight = _weight_grad(payloads, src, grad2d.contiguous()).to(weight.dtype)
     if need_payload:
         grad_read = torch.matmul(grad2d, weight).reshape(B, T, C, 1, P).contiguous()
         grad_payload = _ops.latest_k_backward(src.view(B, T, C, 1), grad_read, ctx.chain)

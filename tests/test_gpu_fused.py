@@ -123,3 +123,45 @@ def test_fused_latest1_linear_gradients(device, dtype, M):
     tol = 2e-2 if dtype == torch.bfloat16 else 1e-5
     assert (gp - p64.grad).abs().max() <= tol * p64.grad.abs().max() + 1e-6
     assert (gw - W64.grad).abs().max() <= tol * W64.grad.abs().max() + 1e-6
+
+
+# B, T, C, P, M, dtype, share of slots without a source: row counts around the
+# 64-row steps and the row ranges, every result-tile height (M up to 64, 128,
+# 192, 256, beyond), partial column tiles (C*P not a multiple of 256)
+WGRAD = [
+    (1, 1, 1, 8, 8, torch.bfloat16, 0.0),
+    (1, 63, 3, 24, 40, torch.float16, 0.5),
+    (1, 64, 4, 64, 64, torch.bfloat16, 0.3),
+    (1, 65, 5, 56, 72, torch.bfloat16, 0.6),
+    (2, 641, 2, 128, 128, torch.float16, 0.2),
+    (3, 999, 16, 64, 192, torch.bfloat16, 0.6),
+    (1, 2049, 33, 8, 256, torch.bfloat16, 0.1),
+    (1, 513, 3, 16, 520, torch.float16, 0.9),
+    (1, 300, 2, 16, 64, torch.bfloat16, 1.0),
+    (1, 300, 2, 16, 12, torch.bfloat16, 0.5),  # M not whole units: the library product
+]
+
+
+@pytest.mark.parametrize("case", WGRAD, ids=[str(i) for i in range(len(WGRAD))])
+def test_weight_gradient_of_looked_up_rows(device, case):
+    """gw = grad^T x rows against fp64: exact products, fp32 sums in any order
+    (<= n 2^-24 of the sum of magnitudes), one rounding to 16 bits."""
+    from ravel_em.fused import _weight_grad
+
+    B, T, C, P, M, dtype, none = case
+    n = B * T
+    g = torch.Generator().manual_seed(T * 7 + M)
+    p = torch.randn(B, T, C, P, generator=g).to(dtype)
+    go = torch.randn(n, M, generator=g).to(dtype)
+    src = torch.randint(0, n * C, (B, T, C), generator=g, dtype=torch.int32)
+    src[torch.rand(B, T, C, generator=g) < none] = -1
+    gw = _weight_grad(p.to(device), src.to(device), go.to(device))
+    again = _weight_grad(p.to(device), src.to(device), go.to(device))
+    s = src.long().view(-1)
+    rows = p.double().view(-1, P)[s.clamp_min(0)] * (s >= 0).view(-1, 1).double()
+    rows = rows.view(n, C * P)
+    ref, scale = go.double().t() @ rows, go.double().abs().t() @ rows.abs()
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    err = (gw.double().cpu() - ref).abs()
+    assert (err <= u * ref.abs() + 1.01 * n * 2.0 ** -24 * scale + 2.0 ** -24).all()
+    assert torch.equal(gw, again)
