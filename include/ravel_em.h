@@ -41,6 +41,7 @@ enum {
   RAVEL_EM_INT32 = 1,
   RAVEL_EM_INT64 = 2,
   RAVEL_EM_ADDR_GEN = 3, /* address code only: addresses produced from a ravel_em_addr_gen */
+  RAVEL_EM_TAPE = 6,     /* address code of ravel_em_latest_k_sum_bwd only: a ravel_em_tape() */
   RAVEL_EM_FLOAT32 = 10,
   RAVEL_EM_BFLOAT16 = 11,
   RAVEL_EM_FLOAT16 = 12,
@@ -363,6 +364,40 @@ int ravel_em_seg_sum_bwd(const void* write_addr, const void* read_addr, int addr
                          int64_t B, int64_t T, int64_t C, int64_t D, int64_t A,
                          void* grad_payload, void* workspace, size_t workspace_bytes,
                          void* stream);
+
+/*
+ * Backward of causal_last_k_lookup, of causal_sum_lookup or of both of one tape
+ * in one pass (the autograd of ravel_memory.py:173-175 and :216-241; the pair is
+ * that of ravel_lm/model.py:366-386):
+ *   grad_payload[s] = sum over the slots (r, j) whose source is s of
+ *                     grad_values[r, j]  +  sum over the later reads r of s's
+ *                     stream of grad_sum[r].
+ * Addresses, mask and k are the forward's.  grad_values [B,T,C,k,D] or
+ * grad_sum [B,T,C,D] may be NULL (no gradient).  Needs no sources.
+ * Deterministic; one rounding of the total.  Takes k <= 8, T <= 2^23 and
+ * gradient rows of one batch row below 2^31 bytes (RAVEL_EM_EINVAL, and a
+ * workspace query of 0, otherwise); any D.  The workspace carries the status
+ * word as the sorting calls' do.
+ *
+ * ravel_em_tape() writes the reads and writes of a call as one compact address
+ * tape of ravel_em_tape_bytes() bytes (8-byte aligned), which the backward takes
+ * in place of the addresses and the mask (addr_dtype RAVEL_EM_TAPE, write_addr
+ * the tape, read_addr and write_mask NULL, has_read 1 in its workspace query):
+ * what a caller keeps between the two passes when the addresses themselves may
+ * change.
+ */
+size_t ravel_em_tape_bytes(int64_t B, int64_t T, int64_t C, int64_t A);
+int ravel_em_tape(const void* write_addr, const void* read_addr, int addr_dtype,
+                  const uint8_t* write_mask, int64_t B, int64_t T, int64_t C, int64_t A,
+                  void* out_tape, void* stream);
+size_t ravel_em_latest_k_sum_bwd_workspace(int64_t B, int64_t T, int64_t C, int64_t D, int64_t A,
+                                           int64_t k, int has_read, int has_mask,
+                                           int payload_dtype);
+int ravel_em_latest_k_sum_bwd(const void* write_addr, const void* read_addr, int addr_dtype,
+                              const uint8_t* write_mask, const void* grad_values,
+                              const void* grad_sum, int payload_dtype, int64_t B, int64_t T,
+                              int64_t C, int64_t D, int64_t A, int64_t k, void* grad_payload,
+                              void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Decode cache, RavelLayerCache (ravel_lm/ravel_memory.py:244-292) with k slots:

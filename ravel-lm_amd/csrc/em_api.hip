@@ -566,6 +566,85 @@ int seg_sum_bwd_run(const AddrIn& wa, const AddrIn* ra, const uint8_t* wmask,
   return RAVEL_EM_OK;
 }
 
+// ------------------------------------------------------- tape walks --
+// Backward of the segmented sum, of the latest-k lookup or of both of one tape
+// in one segmented walk (em_walk.h): reads = writes without a mask walk the
+// tape's own sorted keys, others the sorted tape of reads and writes together.
+// Which of the two, from the call's address arguments.
+struct TapeArgs {
+  AddrIn w, r;
+  bool has_read = false;
+  const uint8_t* wmask = nullptr;
+  bool merged = false;  // w is a merged tape already (RAVEL_EM_TAPE)
+  bool same() const { return !has_read && !wmask && !merged; }
+};
+
+Tape walk_tape(const Tape& tp, bool same) { return same ? tp : merged_tape(tp); }
+
+size_t tape_walk_ws(const Tape& tp, int64_t D, int dtype, int64_t k, bool same) {
+  const Tape wt = walk_tape(tp, same);
+  Bump bp(nullptr);
+  if (wt.wide())
+    take_sort<uint64_t>(bp, wt);
+  else
+    take_sort<uint32_t>(bp, wt);
+  bp.take<uint64_t>(walk_words(tp.nseg(), wt.T, D, dtype, k));
+  return bp.off;
+}
+
+template <typename U>
+int tape_walk_run(const TapeArgs& ta, const Tape& tape, int64_t D, int dtype, bool fwd,
+                  const void* sum_in, const void* val_in, int64_t k, void* out, uint8_t* omask,
+                  void* ws, size_t wsb, hipStream_t s) {
+  const bool same = ta.same();
+  Tape tp = tape;
+  Tape wt = walk_tape(tp, same);
+  Bump bp(ws);
+  SortWs<U> sw = take_sort<U>(bp, wt);
+  tp.status = wt.status = sw.status;
+  const size_t nw = walk_words(tp.nseg(), wt.T, D, dtype, k);
+  uint64_t* words = bp.take<uint64_t>(nw);
+  if (int rc = check_ws(bp, wsb)) return rc;
+  AddrIn in = ta.w;
+  hipError_t e = hipSuccess;
+  if (ta.merged) {
+    in.kind = merged_kind(tp.A);
+  } else if (!same) {
+    // produced addresses decode into the key buffer that the key build fills
+    // last; the merged tape goes into the other, which its first pass overwrites
+    AddrIn wd, rd;
+    const size_t half = (size_t)tp.n() * sizeof(U);
+    e = compact_addresses(ta.w, tp, sw.ka, &wd, s);
+    rd = wd;
+    if (e == hipSuccess && ta.has_read)
+      e = compact_addresses(ta.r, tp, (char*)sw.ka + half, &rd, s);
+    if (e == hipSuccess) e = merge_addresses(wd, rd, ta.wmask, tp, sw.kb, &in, s);
+    if (e != hipSuccess) return hip_fail(e, "merged tape");
+  }
+  U* sorted = nullptr;
+  stage_begin(kStageSort, s);
+  e = sort_call<U>(in, nullptr, wt, sw, &sorted, s, nw ? (uint32_t*)words : nullptr,
+                   2 * (int64_t)nw);
+  stage_end(kStageSort, s);
+  if (e != hipSuccess) return hip_fail(e, "sort");
+  stage_begin(kStageSum, s);
+  e = tape_walk(sorted, sizeof(U) == 8, wt.tbits, same, fwd, tp, D, dtype, sum_in, val_in, k, out,
+                omask, words, s);
+  stage_end(kStageSum, s);
+  if (e != hipSuccess) return hip_fail(e, "segmented walk");
+  return RAVEL_EM_OK;
+}
+
+int tape_walk_call(const TapeArgs& ta, const Tape& tp, int64_t D, int dtype, bool fwd,
+                   const void* sum_in, const void* val_in, int64_t k, void* out, uint8_t* omask,
+                   void* ws, size_t wsb, hipStream_t s) {
+  return walk_tape(tp, ta.same()).wide()
+             ? tape_walk_run<uint64_t>(ta, tp, D, dtype, fwd, sum_in, val_in, k, out, omask, ws,
+                                       wsb, s)
+             : tape_walk_run<uint32_t>(ta, tp, D, dtype, fwd, sum_in, val_in, k, out, omask, ws,
+                                       wsb, s);
+}
+
 template <typename U>
 size_t sum_ws_t(const Tape& tp, int64_t D, int dtype, bool direct, bool backward) {
   Bump bp(nullptr);
@@ -1377,6 +1456,7 @@ size_t ravel_em_seg_sum_bwd_workspace(int64_t B, int64_t T, int64_t C, int64_t D
   const int64_t rows = split_rows(B, T * C);
   const Tape tp = make_tape(B < rows ? B : rows, T, C, A, has_mask != 0, kWrap);
   const bool direct = !has_read && !has_mask;
+  if (walk_applies(tp, D, payload_dtype, 0)) return tape_walk_ws(tp, D, payload_dtype, 0, direct);
   return tp.wide() ? sum_ws_t<uint64_t>(tp, D, payload_dtype, direct, true)
                    : sum_ws_t<uint32_t>(tp, D, payload_dtype, direct, true);
 }
@@ -1410,10 +1490,110 @@ int ravel_em_seg_sum_bwd(const void* write_addr, const void* read_addr, int addr
     const uint8_t* wm = write_mask ? write_mask + b0 * T : nullptr;
     const void* g = at(grad_sum, r0 * row_bytes);
     void* gp = at(grad_payload, r0 * row_bytes);
+    if (walk_applies(t, D, payload_dtype, 0)) {
+      TapeArgs ta;
+      ta.w = w;
+      ta.r = r;
+      ta.has_read = rp != nullptr;
+      ta.wmask = wm;
+      return tape_walk_call(ta, t, D, payload_dtype, false, g, nullptr, 0, gp, nullptr, workspace,
+                            workspace_bytes, s);
+    }
     return t.wide() ? seg_sum_bwd_run<uint64_t>(w, rp, wm, g, payload_dtype, t, D, gp, workspace,
                                                 workspace_bytes, s)
                     : seg_sum_bwd_run<uint32_t>(w, rp, wm, g, payload_dtype, t, D, gp, workspace,
                                                 workspace_bytes, s);
+  });
+}
+
+size_t ravel_em_tape_bytes(int64_t B, int64_t T, int64_t C, int64_t A) {
+  if (check_tape(B, T, C, A)) return 0;
+  return merged_bytes(make_tape(B, T, C, A, true, kWrap));
+}
+
+int ravel_em_tape(const void* write_addr, const void* read_addr, int addr_dtype,
+                  const uint8_t* write_mask, int64_t B, int64_t T, int64_t C, int64_t A,
+                  void* out_tape, void* stream) {
+  g_err.clear();
+  if (int rc = check_tape(B, T, C, A)) return rc;
+  if (int rc = check_addr_dtype(addr_dtype, false)) return rc;
+  const Tape tp = make_tape(B, T, C, A, write_mask != nullptr, kWrap);
+  if (tp.n() == 0) return RAVEL_EM_OK;
+  if (!write_addr || !out_tape) return fail(RAVEL_EM_EINVAL, "null pointer");
+  if ((uintptr_t)out_tape % 8) return fail(RAVEL_EM_EINVAL, "the tape must be 8-byte aligned");
+  AddrIn w, r, out;
+  w.kind = r.kind = addr_dtype;
+  w.dense = write_addr;
+  r.dense = read_addr ? read_addr : write_addr;
+  const hipError_t e = merge_addresses(w, r, write_mask, tp, out_tape, &out, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "merged tape");
+  return RAVEL_EM_OK;
+}
+
+size_t ravel_em_latest_k_sum_bwd_workspace(int64_t B, int64_t T, int64_t C, int64_t D, int64_t A,
+                                           int64_t k, int has_read, int has_mask,
+                                           int payload_dtype) {
+  if (k < 1 || D < 1 || check_rows(B, T, C, A, k)) return 0;
+  const int64_t rows = split_rows(B, T * C * k);
+  const Tape tp = make_tape(B < rows ? B : rows, T, C, A, has_mask != 0, kWrap);
+  if (tp.n() == 0) return kStatusBytes;
+  if (!walk_applies(tp, D, payload_dtype, k)) return 0;
+  return tape_walk_ws(tp, D, payload_dtype, k, !has_read && !has_mask);
+}
+
+int ravel_em_latest_k_sum_bwd(const void* write_addr, const void* read_addr, int addr_dtype,
+                              const uint8_t* write_mask, const void* grad_values,
+                              const void* grad_sum, int payload_dtype, int64_t B, int64_t T,
+                              int64_t C, int64_t D, int64_t A, int64_t k, void* grad_payload,
+                              void* workspace, size_t workspace_bytes, void* stream) {
+  g_err.clear();
+  if (k < 1) return fail(RAVEL_EM_EINVAL, "k must be positive");
+  if (int rc = check_rows(B, T, C, A, k)) return rc;
+  const bool merged = addr_dtype == RAVEL_EM_TAPE;
+  if (!merged)
+    if (int rc = check_addr_dtype(addr_dtype)) return rc;
+  if (merged && (read_addr || write_mask))
+    return fail(RAVEL_EM_EINVAL, "a tape already holds its reads and its mask");
+  if (int rc = check_payload_dtype(payload_dtype)) return rc;
+  if (D < 1) return fail(RAVEL_EM_EINVAL, "payload dim must be >= 1");
+  const Tape tp = make_tape(B, T, C, A, write_mask != nullptr, kWrap);
+  if (tp.n() == 0) return clear_status(workspace, workspace_bytes, stream);
+  if (!write_addr || (!grad_values && !grad_sum) || !grad_payload)
+    return fail(RAVEL_EM_EINVAL, "null pointer");
+  AddrPair ap;
+  if (merged) {
+    ap.w.kind = merged_kind(A);
+    ap.w.dense = write_addr;
+  } else if (int rc = addr_pair(write_addr, read_addr, addr_dtype, C, &ap)) {
+    return rc;
+  }
+  hipStream_t s = (hipStream_t)stream;
+  const int64_t row_bytes = D * dtype_size(payload_dtype);
+  const int64_t rows = split_rows(B, T * C * k);
+  Tape most = tp;
+  most.B = B < rows ? B : rows;
+  if (!walk_applies(most, D, payload_dtype, k))
+    return fail(RAVEL_EM_EINVAL,
+                "the joint backward takes k <= 8, T <= 2^23 and T*C*k*D elements of one batch "
+                "row below 2^31 bytes (T=%lld C=%lld D=%lld k=%lld)",
+                (long long)T, (long long)C, (long long)D, (long long)k);
+  return split_batch(B, rows, workspace, workspace_bytes, s, [&](int64_t nb, int64_t b0) -> int {
+    Tape t = tp;
+    t.B = nb;
+    const int64_t r0 = b0 * T * C;
+    TapeArgs ta;
+    ta.merged = merged;
+    if (merged) {
+      ta.w.dense = at(ap.w.dense, b0 * (int64_t)(merged_bytes(tp) / (size_t)B));
+    } else {
+      ta.w = addr_rows(ap.w, b0, T, C);
+      ta.has_read = ap.rp != nullptr;
+      if (ap.rp) ta.r = addr_rows(*ap.rp, b0, T, C);
+      ta.wmask = write_mask ? write_mask + b0 * T : nullptr;
+    }
+    return tape_walk_call(ta, t, D, payload_dtype, false, at(grad_sum, r0 * row_bytes),
+                          at(grad_values, r0 * k * row_bytes), k, at(grad_payload, r0 * row_bytes),
+                          nullptr, workspace, workspace_bytes, s);
   });
 }
 

@@ -353,6 +353,25 @@ hipError_t seg_sum_bwd(const U* sorted, const int32_t* spos, const void* grad_ou
                        uint8_t* flag, void* carry, uint64_t* walk, void* grad_payload,
                        hipStream_t s);
 
+// Segmented walk of a sorted tape (em_walk.h): fwd false, the backward (out =
+// per-write gradient from sum_in [B,T,C,D] and / or val_in [B,T,C,k,D]); fwd true,
+// the forward sum (out, omask from sum_in = payload).  keys: same (reads at the
+// write addresses, no mask) the tape's sorted keys, else those of
+// merged_tape(tp), tbits its tape's; words: walk_words() words, zero on entry.
+bool walk_applies(const Tape& tp, int64_t D, int dtype, int64_t k);
+size_t walk_words(int64_t nseg, int64_t L, int64_t D, int dtype, int64_t k);
+hipError_t tape_walk(const void* keys, bool wide, int tbits, bool same, bool fwd, const Tape& tp,
+                     int64_t D, int dtype, const void* sum_in, const void* val_in, int64_t k,
+                     void* out, uint8_t* omask, uint64_t* words, hipStream_t s);
+// Reads and writes of a tape as one address tensor [B,2T,C] (even steps the
+// reads, odd the writes, a masked write the address A) in buf (merged_bytes()),
+// and the tape that sorts it.  wa and ra are dense inputs of one kind.
+Tape merged_tape(const Tape& tp);
+int merged_kind(int64_t A);
+size_t merged_bytes(const Tape& tp);
+hipError_t merge_addresses(const AddrIn& wa, const AddrIn& ra, const uint8_t* wmask, const Tape& tp,
+                           void* buf, AddrIn* out, hipStream_t s);
+
 // Decode cache (values [B*C, A, k, row], filled [B*C, A, k]).
 hipError_t cache_read(const void* values, const uint8_t* filled, const void* addr, bool addr64,
                       int64_t BC, int64_t A, int64_t k, int64_t row_bytes, void* out,

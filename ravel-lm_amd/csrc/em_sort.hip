@@ -1477,25 +1477,21 @@ static hipError_t sort_tape_fused(const AddrIn& addr, const uint8_t* wmask,
   return hipSuccess;
 }
 
-bool sort_short_applies(const Tape& tp);
+bool sort_short_applies(const Tape& tp, bool link);
 template <bool LINK>
 hipError_t seg_sort_short(const AddrIn& addr, const uint8_t* wmask, const Tape& tp, int k,
-                          int32_t* src, uint32_t* keys_out, hipStream_t s);
+                          int32_t* src, uint32_t* keys_out, hipStream_t s,
+                          uint32_t* zero = nullptr, int64_t zero_words = 0);
 
 template <typename U>
 hipError_t sort_tape(const AddrIn& addr, const uint8_t* wmask, const Tape& tp, U* ka,
                      U* kb, uint32_t* counts, U** sorted, hipStream_t s, uint32_t* zero,
                      int64_t zero_words, int32_t* link_seg) {
   if (!tp.status) return hipErrorInvalidValue;  // every sort clears and may set the call's word
-  if (sizeof(U) == 4 && tp.fused && sort_short_applies(tp)) {
+  if (sizeof(U) == 4 && tp.fused && sort_short_applies(tp, link_seg != nullptr) && tp.n() > 0) {
     // short tapes: each segment sorted in LDS by one block (the caller links)
-    if (zero && zero_words > 0) {
-      const hipError_t ez = fill_bytes(zero, 0, (size_t)zero_words * 4, s);
-      if (ez != hipSuccess) return ez;
-    }
     *sorted = ka;
-    if (tp.n() == 0) return hipSuccess;
-    return seg_sort_short<false>(addr, wmask, tp, 0, nullptr, (uint32_t*)ka, s);
+    return seg_sort_short<false>(addr, wmask, tp, 0, nullptr, (uint32_t*)ka, s, zero, zero_words);
   }
   if (tp.fused) {
     const PackPlan pl = fused_plan(tp, sizeof(U));
@@ -1581,13 +1577,17 @@ template <typename AS, int ITEMS, bool LINK, int NT>
 __global__ __launch_bounds__(NT) void seg_sort_link_kernel(
     const AS addr, const uint8_t* __restrict__ wmask, int64_t T, int64_t C, int64_t A, int tbits,
     int npass, int mode, int trunc32, int k, int64_t nseg, int32_t* __restrict__ src,
-    uint32_t* __restrict__ keys_out, uint32_t* __restrict__ status) {
+    uint32_t* __restrict__ keys_out, uint32_t* __restrict__ status, uint32_t* __restrict__ zero,
+    int64_t zero_words) {
   constexpr int NW = NT / kWave;
   __shared__ uint32_t wcnt[NW][kRadix];
   __shared__ uint32_t dstart[kRadix];
   __shared__ uint32_t scan_tmp[NW + 1];
-  __shared__ uint32_t buf[2][kShortT];
-  __shared__ uint16_t inv[kShortT];
+  // one buffer: a pass's keys are all in registers before any is written back
+  // (rank_tile's barriers stand between), so no second one is needed
+  __shared__ uint32_t sorted[NT * ITEMS];
+  __shared__ uint16_t inv[LINK ? NT * ITEMS : 2];
+  zero_slice(zero, zero_words);  // state of later kernels; every block, padding included
   const int tid = threadIdx.x, w = tid / kWave, lane = tid % kWave;
   if (blockIdx.x == 0 && tid == 0) *status = 0;  // the call's first sort kernel
   const int64_t seg = xcd_block(blockIdx.x, gridDim.x);
@@ -1610,14 +1610,12 @@ __global__ __launch_bounds__(NT) void seg_sort_link_kernel(
     if (wmask && t < n && !wmask[b * T + t]) a = A;
     key[i] = t < n ? ((uint32_t)a << tbits) | (uint32_t)t : 0u;
   }
-  uint32_t* sorted = buf[0];
   for (int p = 0; p < npass; ++p) {
     const int shift = tbits + 8 * p;
     uint32_t rank[ITEMS];
     uint32_t own;
     rank_tile<uint32_t, ITEMS, NT>(n, shift, wcnt, dstart, scan_tmp, key, rank, &own);
     __syncthreads();  // dstart of every digit
-    sorted = buf[p & 1];
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
       const int idx = w * kWave * ITEMS + i * kWave + lane;
@@ -1687,7 +1685,8 @@ __global__ __launch_bounds__(NT) void seg_sort_link_kernel(
 
 template <bool LINK>
 hipError_t seg_sort_short(const AddrIn& addr, const uint8_t* wmask, const Tape& tp, int k,
-                          int32_t* src, uint32_t* keys_out, hipStream_t s) {
+                          int32_t* src, uint32_t* keys_out, hipStream_t s, uint32_t* zero,
+                          int64_t zero_words) {
   const unsigned grid = xcd_grid(tp.nseg(), 1, (int64_t)1 << 31);
   const int npass = (tp.abits + 7) / 8;
   return with_addr(addr, tp, [&](auto a) {
@@ -1695,24 +1694,29 @@ hipError_t seg_sort_short(const AddrIn& addr, const uint8_t* wmask, const Tape& 
 #define REM_SL(IT)                                                                            \
   seg_sort_link_kernel<decltype(a), IT, LINK, kShortThreads><<<grid, kShortThreads, 0, s>>>(   \
       a, wmask, tp.T, tp.C, tp.A, tp.tbits, npass, tp.mode, tp.trunc32 ? 1 : 0, k, tp.nseg(), \
-      src, keys_out, tp.status)
+      src, keys_out, tp.status, zero, zero_words)
     if (tp.T <= kShortThreads)
       REM_SL(1);
     else if (tp.T <= 2 * kShortThreads)
       REM_SL(2);
-    else
+    else if (LINK || tp.T <= 4 * kShortThreads)
       REM_SL(4);
+    else
+      REM_SL(LINK ? 4 : 8);
 #undef REM_SL
     return hipGetLastError();
   });
 }
 
-bool sort_short_applies(const Tape& tp) {
-  return tp.T >= 1 && tp.T <= kShortT && !tp.wide() && (tp.abits + 7) / 8 <= 4;
+// Segments that one block sorts in LDS.  Keys alone go up to twice the length of
+// the links, whose global sort ends in a linking pass instead of a sorted one.
+bool sort_short_applies(const Tape& tp, bool link) {
+  return tp.T >= 1 && tp.T <= (link ? kShortT : 2 * kShortT) && !tp.wide() &&
+         (tp.abits + 7) / 8 <= 4;
 }
 
 bool link_short_applies(const Tape& tp, int64_t k) {
-  return !tp.masked && sort_short_applies(tp) && k >= 1 && tp.n() * k < ((int64_t)1 << 31);
+  return !tp.masked && sort_short_applies(tp, true) && k >= 1 && tp.n() * k < ((int64_t)1 << 31);
 }
 
 hipError_t link_short(const AddrIn& addr, const Tape& tp, int k, int32_t* src, hipStream_t s) {

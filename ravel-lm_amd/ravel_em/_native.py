@@ -18,6 +18,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
 # dtype codes (include/ravel_em.h)
 INT32, INT64 = 1, 2
 ADDR_GEN = 3  # address code: write/read pointers are AddrGen descriptors
+TAPE = 6  # address code of the joint backward: write pointer is a merged tape
 FLOAT32, BFLOAT16, FLOAT16, FLOAT64 = 10, 11, 12, 13
 
 _PAYLOAD_CODES = {
@@ -99,6 +100,15 @@ SIGNATURES = {
     "ravel_em_seg_sum_bwd_workspace": (_sz, [_i64, _i64, _i64, _i64, _i64, _i, _i, _i]),
     "ravel_em_seg_sum_bwd": (
         _i, [_vp, _vp, _i, _vp, _vp, _i, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _sz, _vp]
+    ),
+    "ravel_em_tape_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "ravel_em_tape": (_i, [_vp, _vp, _i, _vp, _i64, _i64, _i64, _i64, _vp, _vp]),
+    "ravel_em_latest_k_sum_bwd_workspace": (
+        _sz, [_i64, _i64, _i64, _i64, _i64, _i64, _i, _i, _i]
+    ),
+    "ravel_em_latest_k_sum_bwd": (
+        _i,
+        [_vp, _vp, _i, _vp, _vp, _vp, _i, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _sz, _vp],
     ),
     "ravel_em_cache_read": (_i, [_vp, _vp, _vp, _i, _i, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp]),
     "ravel_em_cache_write": (_i, [_vp, _vp, _vp, _i, _vp, _i, _i64, _i64, _i64, _i64, _i64, _vp]),

@@ -126,12 +126,15 @@ def _latest_k_setup(ctx, inputs, output):
     ctx.chain = read_addresses is None and write_mask is None
     ctx.want_src = want_src
     ctx.mark_non_differentiable(mask, src)
+    ctx.set_materialize_grads(False)  # no zero gradients of the mask and the sources
 
 
 def _latest_k_grad(ctx, grad_values, _grad_mask, _grad_src):
     (src,) = ctx.saved_tensors
     if not ctx.want_src:
         raise RuntimeError("ravel_em.latest_k was called without sources; cannot differentiate")
+    if grad_values is None:
+        return (None,) * 7
     grad_payload = latest_k_backward(src, grad_values, ctx.chain)
     return None, grad_payload, None, None, None, None, None
 
@@ -226,10 +229,13 @@ def _seg_sum_setup(ctx, inputs, output):
     ctx.save_for_backward(write_addresses, read_addresses, write_mask)
     ctx.address_space = address_space
     ctx.mark_non_differentiable(output[1])
+    ctx.set_materialize_grads(False)
 
 
 def _seg_sum_grad(ctx, grad_sum, _grad_mask):
     write_addresses, read_addresses, write_mask = ctx.saved_tensors
+    if grad_sum is None:
+        return (None,) * 5
     grad_payload = seg_sum_backward(write_addresses, read_addresses, write_mask, grad_sum, ctx.address_space)
     return None, grad_payload, None, None, None
 
@@ -305,6 +311,58 @@ def _latest_k_sum_fake(write_addresses, payloads, read_addresses, write_mask, ad
     )
 
 
+def joint_backward_applies(T: int, C: int, D: int, k: int, element_size: int) -> bool:
+    """Whether latest_k_sum_backward (one walk, no sources) takes the shape: the
+    library's own rule (its workspace query is not 0), in plain arithmetic that
+    torch.compile can trace."""
+    step = C * D * element_size * k  # gradient bytes of one time step
+    return (1 <= k <= 8 and 1 <= T <= 1 << 23 and C * k < 1 << 24 and step < 1 << 24
+            and T * step < 1 << 31)
+
+
+@torch.library.custom_op("ravel_em::latest_k_sum_backward", mutates_args=())
+def latest_k_sum_backward(
+    write_addresses: Tensor,
+    read_addresses: Optional[Tensor],
+    write_mask: Optional[Tensor],
+    grad_values: Optional[Tensor],
+    grad_sum: Optional[Tensor],
+    address_space: int,
+    k: int,
+    taped: bool,
+) -> Tensor:
+    """Payload gradient of latest_k (grad_values [B,T,C,k,D]), of seg_sum
+    (grad_sum [B,T,C,D]) or of both of one tape; with ``taped`` the first
+    argument is the tape that latest_k_taped returned."""
+    lib = nat.library()
+    gv = None if grad_values is None else grad_values.contiguous()
+    gs = None if grad_sum is None else grad_sum.contiguous()
+    g = gs if gv is None else gv
+    B, T, C, D = g.shape[0], g.shape[1], g.shape[2], g.shape[-1]
+    grad_payload = g.new_empty(B, T, C, D)
+    code = nat.payload_code(g.dtype)
+    nbytes = lib.ravel_em_latest_k_sum_bwd_workspace(
+        B, T, C, D, address_space, k, int(taped or read_addresses is not None),
+        int(write_mask is not None), code)
+    ws = nat.workspace(nbytes, g.device)
+    _call(
+        lib.ravel_em_latest_k_sum_bwd,
+        nat.ptr(write_addresses), nat.ptr(read_addresses),
+        nat.TAPE if taped else nat.addr_code(write_addresses.dtype), nat.ptr(write_mask),
+        nat.ptr(gv), nat.ptr(gs), code, B, T, C, D, address_space, k, nat.ptr(grad_payload),
+        nat.ptr(ws), ws.numel(), nat.stream_of(g),
+    )
+    nat.after_call(ws)
+    return grad_payload
+
+
+@latest_k_sum_backward.register_fake
+def _latest_k_sum_backward_fake(write_addresses, read_addresses, write_mask, grad_values, grad_sum,
+                                address_space, k, taped):
+    g = grad_sum if grad_values is None else grad_values
+    return g.new_empty(*g.shape[:3], g.shape[-1])
+
+
 def _latest_k_sum_setup(ctx, inputs, output):
     write_addresses, payloads, read_addresses, write_mask, address_space, k, want_src = inputs
     _, mask, src, _, smask = output
@@ -312,20 +370,101 @@ def _latest_k_sum_setup(ctx, inputs, output):
     ctx.chain = read_addresses is None and write_mask is None
     ctx.want_src = want_src
     ctx.address_space = address_space
+    ctx.k = k
     ctx.mark_non_differentiable(mask, src, smask)
+    ctx.set_materialize_grads(False)
 
 
 def _latest_k_sum_grad(ctx, grad_values, _grad_mask, _grad_src, grad_sum, _grad_smask):
     src, write_addresses, read_addresses, write_mask = ctx.saved_tensors
-    if not ctx.want_src:
-        raise RuntimeError("ravel_em.latest_k_sum was called without sources; cannot differentiate")
-    grad_payload = latest_k_backward(src, grad_values, ctx.chain)
-    grad_payload = grad_payload + seg_sum_backward(write_addresses, read_addresses, write_mask,
-                                                   grad_sum, ctx.address_space)
+    if grad_values is None and grad_sum is None:
+        return (None,) * 7
+    g = grad_sum if grad_values is None else grad_values
+    B, T, C, D = g.shape[0], g.shape[1], g.shape[2], g.shape[-1]
+    if joint_backward_applies(T, C, D, ctx.k, g.element_size()):
+        grad_payload = latest_k_sum_backward(write_addresses, read_addresses, write_mask,
+                                             grad_values, grad_sum, ctx.address_space, ctx.k, False)
+        return None, grad_payload, None, None, None, None, None
+    grad_payload = None
+    if grad_values is not None:
+        if not ctx.want_src:
+            raise RuntimeError("ravel_em.latest_k_sum was called without sources; "
+                               "cannot differentiate")
+        grad_payload = latest_k_backward(src, grad_values, ctx.chain)
+    if grad_sum is not None:
+        gs = seg_sum_backward(write_addresses, read_addresses, write_mask, grad_sum,
+                              ctx.address_space)
+        grad_payload = gs if grad_payload is None else grad_payload + gs
     return None, grad_payload, None, None, None, None, None
 
 
 latest_k_sum.register_autograd(_latest_k_sum_grad, setup_context=_latest_k_sum_setup)
+
+
+# ------------------------------------------- latest-k with its own tape --
+
+
+def _tape_dtype(address_space: int) -> torch.dtype:
+    """Storage type of a merged tape (the kernels' unsigned kind of that size)."""
+    if address_space < 1 << 16:
+        return torch.int16
+    return torch.int32 if address_space < 1 << 32 else torch.int64
+
+
+@torch.library.custom_op("ravel_em::latest_k_taped", mutates_args=())
+def latest_k_taped(
+    write_addresses: Tensor,
+    payloads: Tensor,
+    read_addresses: Optional[Tensor],
+    write_mask: Optional[Tensor],
+    address_space: int,
+    k: int,
+) -> Tuple[Tensor, Tensor, Tensor]:
+    """latest_k for a training step with separate reads or a write mask: values,
+    mask and the compact tape of its reads and writes ([B, 2T, C]), from which
+    the backward sorts again.  The tape is a copy, so the addresses may change
+    between the passes, and smaller than k sources a record."""
+    lib = nat.library()
+    B, T, C = write_addresses.shape
+    values, mask, _ = latest_k_impl(write_addresses, payloads, read_addresses, write_mask,
+                                    address_space, k, False)
+    tape = torch.empty(B, 2 * T, C, dtype=_tape_dtype(address_space), device=payloads.device)
+    _call(
+        lib.ravel_em_tape, nat.ptr(write_addresses), nat.ptr(read_addresses),
+        nat.addr_code(write_addresses.dtype), nat.ptr(write_mask), B, T, C, address_space,
+        nat.ptr(tape), nat.stream_of(payloads),
+    )
+    return values, mask, tape
+
+
+@latest_k_taped.register_fake
+def _latest_k_taped_fake(write_addresses, payloads, read_addresses, write_mask, address_space, k):
+    B, T, C = write_addresses.shape
+    return (
+        payloads.new_empty(B, T, C, k, payloads.shape[-1]),
+        torch.empty(B, T, C, k, dtype=torch.bool, device=payloads.device),
+        torch.empty(B, 2 * T, C, dtype=_tape_dtype(address_space), device=payloads.device),
+    )
+
+
+def _latest_k_taped_setup(ctx, inputs, output):
+    _, mask, tape = output
+    ctx.save_for_backward(tape)
+    ctx.address_space, ctx.k = inputs[4], inputs[5]
+    ctx.mark_non_differentiable(mask, tape)
+    ctx.set_materialize_grads(False)
+
+
+def _latest_k_taped_grad(ctx, grad_values, _grad_mask, _grad_tape):
+    (tape,) = ctx.saved_tensors
+    if grad_values is None:
+        return (None,) * 6
+    grad_payload = latest_k_sum_backward(tape, None, None, grad_values, None, ctx.address_space,
+                                         ctx.k, True)
+    return None, grad_payload, None, None, None, None
+
+
+latest_k_taped.register_autograd(_latest_k_taped_grad, setup_context=_latest_k_taped_setup)
 
 
 # ------------------------------------------------------- direct C calls --

@@ -309,10 +309,13 @@ def _latest_k_gen_setup(ctx, inputs, output):
     ctx.chain = read_logits is None and write_mask is None
     ctx.want_src = want_src
     ctx.mark_non_differentiable(mask, src)
+    ctx.set_materialize_grads(False)
 
 
 def _latest_k_gen_grad(ctx, grad_values, _grad_mask, _grad_src):
     (src,) = ctx.saved_tensors
+    if grad_values is None:
+        return (None,) * 15
     if not ctx.want_src:
         raise RuntimeError("ravel_em.latest_k_gen was called without sources; cannot differentiate")
     grad_payload = _ops.latest_k_backward(src, grad_values, ctx.chain)
@@ -388,10 +391,13 @@ def _seg_sum_gen_setup(ctx, inputs, output):
     ctx.save_for_backward(tokens, history, write_logits, read_logits, write_mask)
     ctx.cfg = inputs[6:]
     ctx.mark_non_differentiable(output[1])
+    ctx.set_materialize_grads(False)
 
 
 def _seg_sum_gen_grad(ctx, grad_sum, _grad_mask):
     tokens, history, write_logits, read_logits, write_mask = ctx.saved_tensors
+    if grad_sum is None:
+        return (None,) * 13
     grad_payload = seg_sum_gen_backward(tokens, history, write_logits, read_logits, write_mask,
                                         grad_sum, *ctx.cfg)
     return (None, None, None, None, grad_payload) + (None,) * 8
@@ -442,25 +448,76 @@ def _latest_k_sum_gen_fake(tokens, history, write_logits, read_logits, payloads,
             torch.empty(B, T, C, dtype=torch.bool, device=dev))
 
 
+@torch.library.custom_op("ravel_em::latest_k_sum_gen_backward", mutates_args=())
+def latest_k_sum_gen_backward(tokens: Optional[Tensor], history: Optional[Tensor],
+                              write_logits: Optional[Tensor], read_logits: Optional[Tensor],
+                              write_mask: Optional[Tensor], grad_values: Optional[Tensor],
+                              grad_sum: Optional[Tensor], n_literal: int, bos: int,
+                              n_learned: int, ncb: int, cbs: int, position: int,
+                              address_space: int, k: int) -> Tensor:
+    """_ops.latest_k_sum_backward with the addresses produced in the kernels."""
+    lib = nat.library()
+    gv = None if grad_values is None else grad_values.contiguous()
+    gs = None if grad_sum is None else grad_sum.contiguous()
+    g = gs if gv is None else gv
+    B, T, C, D = g.shape[0], g.shape[1], g.shape[2], g.shape[-1]
+    grad_payload = g.new_empty(B, T, C, D)
+    code = nat.payload_code(g.dtype)
+    w, r = _descs(tokens, history, write_logits, read_logits, n_literal, bos, n_learned, ncb, cbs,
+                  position)
+    nbytes = lib.ravel_em_latest_k_sum_bwd_workspace(B, T, C, D, address_space, k,
+                                                     int(r is not None),
+                                                     int(write_mask is not None), code)
+    ws = nat.workspace(nbytes, g.device)
+    nat.check(lib.ravel_em_latest_k_sum_bwd(
+        nat.ref(w), nat.ref(r), nat.ADDR_GEN, nat.ptr(write_mask), nat.ptr(gv), nat.ptr(gs), code,
+        B, T, C, D, address_space, k, nat.ptr(grad_payload), nat.ptr(ws), ws.numel(),
+        nat.stream_of(g)))
+    nat.after_call(ws)
+    return grad_payload
+
+
+@latest_k_sum_gen_backward.register_fake
+def _latest_k_sum_gen_backward_fake(tokens, history, write_logits, read_logits, write_mask,
+                                    grad_values, grad_sum, n_literal, bos, n_learned, ncb, cbs,
+                                    position, address_space, k):
+    g = grad_sum if grad_values is None else grad_values
+    return g.new_empty(*g.shape[:3], g.shape[-1])
+
+
 def _latest_k_sum_gen_setup(ctx, inputs, output):
     tokens, history, write_logits, read_logits, _payloads, write_mask = inputs[:6]
     _, mask, src, _, smask = output
     ctx.save_for_backward(src, tokens, history, write_logits, read_logits, write_mask)
     ctx.chain = read_logits is None and write_mask is None
-    ctx.want_src = inputs[-1]
+    ctx.k, ctx.want_src = inputs[-2], inputs[-1]
     ctx.cfg = inputs[6:13]
     ctx.mark_non_differentiable(mask, src, smask)
+    ctx.set_materialize_grads(False)
 
 
 def _latest_k_sum_gen_grad(ctx, grad_values, _grad_mask, _grad_src, grad_sum, _grad_smask):
     src, tokens, history, write_logits, read_logits, write_mask = ctx.saved_tensors
-    if not ctx.want_src:
-        raise RuntimeError("ravel_em.latest_k_sum_gen was called without sources; "
-                           "cannot differentiate")
-    grad_payload = _ops.latest_k_backward(src, grad_values, ctx.chain)
-    grad_payload = grad_payload + seg_sum_gen_backward(tokens, history, write_logits, read_logits,
-                                                       write_mask, grad_sum, *ctx.cfg)
-    return (None, None, None, None, grad_payload) + (None,) * 10
+    rest = (None,) * 10
+    if grad_values is None and grad_sum is None:
+        return (None,) * 5 + rest
+    g = grad_sum if grad_values is None else grad_values
+    B, T, C, D = g.shape[0], g.shape[1], g.shape[2], g.shape[-1]
+    if _ops.joint_backward_applies(T, C, D, ctx.k, g.element_size()):
+        grad_payload = latest_k_sum_gen_backward(tokens, history, write_logits, read_logits,
+                                                 write_mask, grad_values, grad_sum, *ctx.cfg, ctx.k)
+        return (None, None, None, None, grad_payload) + rest
+    grad_payload = None
+    if grad_values is not None:
+        if not ctx.want_src:
+            raise RuntimeError("ravel_em.latest_k_sum_gen was called without sources; "
+                               "cannot differentiate")
+        grad_payload = _ops.latest_k_backward(src, grad_values, ctx.chain)
+    if grad_sum is not None:
+        gs = seg_sum_gen_backward(tokens, history, write_logits, read_logits, write_mask, grad_sum,
+                                  *ctx.cfg)
+        grad_payload = gs if grad_payload is None else grad_payload + gs
+    return (None, None, None, None, grad_payload) + rest
 
 
 latest_k_sum_gen.register_autograd(_latest_k_sum_gen_grad, setup_context=_latest_k_sum_gen_setup)
@@ -521,7 +578,10 @@ def last_k_and_sum_lookup(src: LayerAddresses, payloads: Tensor, *, address_spac
     tok, hist, wl, rl = src.tensors()
     nat.require_device(payloads, tok, hist, wl, rl, write_mask)
     m = None if write_mask is None else write_mask.bool().contiguous()
-    want_src = torch.is_grad_enabled() and payloads.requires_grad
+    # the sources are kept only for the shapes whose backward needs them
+    want_src = (torch.is_grad_enabled() and payloads.requires_grad
+                and not _ops.joint_backward_applies(*payloads.shape[1:], int(k),
+                                                    payloads.element_size()))
     values, mask, _, summed, sum_mask = latest_k_sum_gen(
         tok, hist, wl, rl, payloads.contiguous(), m, *src.cfg(), int(address_space), int(k),
         bool(want_src))

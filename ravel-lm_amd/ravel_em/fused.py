@@ -118,6 +118,7 @@ def _setup(ctx, inputs, output):
     ctx.save_for_backward(src, payloads, weight)
     ctx.chain = read_addresses is None
     ctx.mark_non_differentiable(src)
+    ctx.set_materialize_grads(False)  # no zero gradient of the sources
 
 
 def _grads(ctx, grad_out, need_payload: bool, need_weight: bool):
@@ -137,6 +138,8 @@ def _grads(ctx, grad_out, need_payload: bool, need_weight: bool):
 
 
 def _backward(ctx, grad_out, _grad_src):
+    if grad_out is None:
+        return (None,) * 5
     gp, gw = _grads(ctx, grad_out, ctx.needs_input_grad[1], ctx.needs_input_grad[3])
     return None, gp, None, gw, None
 
@@ -191,9 +194,12 @@ def _setup_gen(ctx, inputs, output):
     ctx.save_for_backward(src, payloads, weight)
     ctx.chain = inputs[3] is None
     ctx.mark_non_differentiable(src)
+    ctx.set_materialize_grads(False)
 
 
 def _backward_gen(ctx, grad_out, _grad_src):
+    if grad_out is None:
+        return (None,) * 13
     gp, gw = _grads(ctx, grad_out, ctx.needs_input_grad[4], ctx.needs_input_grad[5])
     return (None, None, None, None, gp, gw) + (None,) * 7
 

@@ -132,6 +132,10 @@ def causal_last_k_lookup(
     m = None if write_mask is None else write_mask.bool().contiguous()
     want_src = torch.is_grad_enabled() and payloads.requires_grad
     p = payloads.contiguous()
+    if want_src and (r is not None or m is not None) and _ops.joint_backward_applies(
+            T, C, p.shape[-1], int(k), p.element_size()):
+        values, mask, _ = _ops.latest_k_taped(w, p, r, m, int(address_space), int(k))
+        return values, mask
     op = _ops.latest_k_impl if not want_src and _ops.eager(w, p, r, m) else _ops.latest_k
     values, mask, _ = op(w, p, r, m, int(address_space), int(k), want_src)
     return values, mask
@@ -267,7 +271,10 @@ def causal_last_k_and_sum_lookup(
     p = payloads.contiguous()
     graph = torch.is_grad_enabled() and p.requires_grad
     op = _ops.latest_k_sum_impl if not graph and _ops.eager(w, p, r, m) else _ops.latest_k_sum
-    values, mask, _, summed, sum_mask = op(w, p, r, m, int(address_space), int(k), graph)
+    # the sources are kept only for the shapes whose backward needs them
+    want_src = graph and not _ops.joint_backward_applies(T, C, p.shape[-1], int(k),
+                                                         p.element_size())
+    values, mask, _, summed, sum_mask = op(w, p, r, m, int(address_space), int(k), want_src)
     return values, mask, summed, sum_mask
 
 

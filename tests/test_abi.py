@@ -252,3 +252,18 @@ def test_split_hook_and_split_workspaces():
         assert lib.ravel_em_set_split_slots(0) == 0
     assert lib.ravel_em_latest_k_workspace(7, 64, 3, 11, 4, 0, 0, 1) > \
         lib.ravel_em_latest_k_workspace(2, 64, 3, 11, 4, 0, 0, 1)
+
+
+@pytest.mark.parametrize("T,C,D,k", [(1, 1, 1, 1), (4096, 8, 64, 8), (4096, 8, 64, 9), (1 << 23, 1, 1, 1),
+                                     ((1 << 23) + 1, 1, 1, 1), (65536, 16, 128, 8), (65536, 16, 64, 8),
+                                     (3, 1 << 20, 8, 1), (3, 1 << 19, 7, 2), (0, 3, 4, 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64])
+def test_joint_backward_shape_rule_matches_the_library(T, C, D, k, dtype):
+    """The wrapper's rule for the one-walk backward is the library's (its
+    workspace query is 0 exactly where the rule says no)."""
+    from ravel_em import _ops
+
+    n = nat.library().ravel_em_latest_k_sum_bwd_workspace(2, T, C, D, 1000, k, 1, 1,
+                                                          nat.payload_code(dtype))
+    want = _ops.joint_backward_applies(T, C, D, k, torch.empty(0, dtype=dtype).element_size())
+    assert (n > 0) == (want or T == 0)

@@ -143,3 +143,95 @@ def test_sum_gradient(device, case, dtype):
     (want,) = torch.autograd.grad(dense_sum(p64, w, r, A, m), p64, gy.double())
     tol = 1e-5 if dtype == torch.float32 else 2e-2
     torch.testing.assert_close(grad.cpu().double(), want, rtol=tol, atol=tol)
+
+
+# The joint backward (both outputs' gradients in one segmented walk) at the edges
+# of its dispatch: row units of 16, 8, 4 and 2 bytes and several column blocks,
+# every state depth (k = 1, 2, 3..4, 5..8), one item to many parts a segment, runs
+# inside a walker, across walkers and across parts, and stretches of reads with no
+# write for longer than a part.
+JOINT_BWD = [
+    # B, T, C, A, kept share of writes (1 = no mask), separate reads, k, D, dtype
+    (2, 1, 3, 5, 1.0, False, 1, 8, torch.bfloat16),
+    (1, 63, 2, 9, 0.5, True, 2, 24, torch.float16),
+    (3, 257, 2, 300, 1.0, False, 8, 32, torch.float32),
+    (2, 1000, 3, 40, 0.8, True, 4, 64, torch.bfloat16),
+    (1, 1025, 1, 1, 1.0, True, 3, 21, torch.bfloat16),    # one run, 2-byte units
+    (1, 2100, 2, 3, 0.6, False, 5, 50, torch.bfloat16),   # 4-byte units
+    (1, 4097, 2, 700, 1.0, True, 4, 96, torch.bfloat16),  # global sort of the merged tape
+    (1, 4097, 1, 50, 1.0, False, 8, 128, torch.float32),  # several column blocks
+    (1, 3000, 2, 2, 0.7, True, 1, 5, torch.float64),
+    (1, 9000, 1, 1, 0.002, True, 8, 16, torch.float16),   # rare writes: runs of reads
+    (1, 5000, 2, 70000, 1.0, True, 2, 130, torch.float16),  # 32-bit tape
+    (1, 1500, 1, 4, 0.9, True, 7, 300, torch.bfloat16),   # five column blocks of 4-byte units
+]
+
+
+def stream_suffix_sums(write, read, A, mask, grad64):
+    """Per write: the sum of grad64 over the later reads of its stream (fp64)."""
+    B, T, C, D = grad64.shape
+    stream = torch.arange(B).view(B, 1, 1) * C + torch.arange(C)
+    t = torch.arange(T).view(1, T, 1)
+    wk = ((stream * A + write.remainder(A)) * T + t).reshape(-1)
+    rk, order = ((stream * A + read.remainder(A)) * T + t).reshape(-1).sort()
+    csum = torch.cat([torch.zeros(1, D, dtype=torch.float64), grad64.reshape(-1, D)[order].cumsum(0)])
+    lo = torch.searchsorted(rk, wk, right=True)
+    hi = torch.searchsorted(rk, (wk // T + 1) * T)
+    out = (csum[hi] - csum[lo]).view(B, T, C, D)
+    n = (hi - lo).view(B, T, C, 1).double()
+    if mask is not None:
+        out, n = out * mask.view(B, T, 1, 1), n * mask.view(B, T, 1, 1)
+    return out, n
+
+
+@pytest.mark.parametrize("case", JOINT_BWD, ids=[str(i) for i in range(len(JOINT_BWD))])
+def test_joint_gradient(device, case):
+    """|err| <= u |x| (one rounding) + n 2^-24 (2^-52 for fp32/fp64 rows) sum|terms|:
+    a sum of n terms in any order; the reference's own cumulative sums add
+    T 2^-52 of theirs."""
+    from ravel_em import causal_last_k_and_sum_lookup
+
+    B, T, C, A, keep, sep, k, D, dtype = case
+    print(f"[joint backward] {case}", flush=True)
+    g = torch.Generator().manual_seed(T + k + D)
+    w = torch.randint(0, A, (B, T, C), generator=g)
+    r = torch.randint(0, A, (B, T, C), generator=g) if sep else None
+    m = (torch.rand(B, T, generator=g) < keep) if keep < 1 else None
+    p = torch.randn(B, T, C, D, generator=g).to(dtype)
+    gv = torch.randn(B, T, C, k, D, generator=g).to(dtype)
+    gs = torch.randn(B, T, C, D, generator=g).to(dtype)
+
+    def run(*which):
+        pg = p.to(device).requires_grad_(True)
+        vals, _, summed, _ = causal_last_k_and_sum_lookup(
+            w.to(device), pg, None if r is None else r.to(device), address_space=A, k=k,
+            write_mask=None if m is None else m.to(device))
+        outs = [(vals, gv), (summed, gs)]
+        (grad,) = torch.autograd.grad([outs[i][0] for i in which], pg,
+                                      [outs[i][1].to(device) for i in which])
+        return grad.cpu()
+
+    src = oracle.latest_k_src(w, r, address_space=A, k=k, write_mask=m)
+    p64 = p.double().requires_grad_(True)
+
+    def lin(x):
+        return torch.autograd.grad(dense_latest_k(p64, src), p64, x)[0]
+
+    rd = w if r is None else r
+    v = (lin(gv.double()), lin(gv.double().abs()), lin(torch.ones_like(gv, dtype=torch.float64)))
+    s64, n = stream_suffix_sums(w, rd, A, m, gs.double())
+    s = (s64, stream_suffix_sums(w, rd, A, m, gs.double().abs())[0], n)
+    wide = dtype in (torch.float32, torch.float64)
+    acc_u = 2.0 ** -52 if wide else 2.0 ** -24
+    u = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24,
+         torch.float64: 2.0 ** -52}[dtype]
+    for which in ((0, 1), (0,), (1,)):
+        got = run(*which)
+        want, scale, terms = (sum(x[i] for j, x in enumerate((v, s)) if j in which) for i in range(3))
+        err = (got.double() - want).abs()
+        bound = u * want.abs() + (1.01 * terms * acc_u + 4 * T * 2.0 ** -52) * scale + \
+            T * 2.0 ** -50 * (1 in which) + 2.0 ** -24 * (not wide)
+        assert (err <= bound).all(), (which, (err / bound).max().item())
+        if which == (0, 1):
+            bits = {2: torch.int16, 4: torch.int32, 8: torch.int64}[got.element_size()]
+            assert torch.equal(got.view(bits), run(0, 1).view(bits)), "two runs differ"
