@@ -339,11 +339,11 @@ int ravel_em_seg_sum_fwd(const void* write_addr, const void* read_addr, int addr
  *   (as ravel_em_seg_sum_fwd).
  * Results equal the two separate calls' (values, masks and sources bit for
  * bit; sums within the same accumulation bound).  The tape is sorted once
- * where one kernel can emit both: tapes of T <= 4096 with k <= 8 (one launch
- * sorts reads and writes in LDS, sums and writes the sources, a second gathers
- * the values) and, for reads = writes without a write_mask and k = 1, longer
- * tapes (one sort, then one walk writes the sums and the latest-1 values);
- * other shapes run the two operators one after the other.  The workspace
+ * where one kernel can emit both: tapes of T <= 4096 with k <= 8 and rows of
+ * whole 16-byte units (one launch sorts reads and writes in LDS, sums and stores
+ * the values) and other tapes with k <= 8 (one sort of reads and writes, then one
+ * segmented walk; out_src costs a resolution of its own there); other shapes run
+ * the two operators one after the other.  The workspace
  * carries the status word as the sorting calls' do.
  */
 size_t ravel_em_latest_k_sum_workspace(int64_t B, int64_t T, int64_t C, int64_t D, int64_t A,
@@ -374,7 +374,7 @@ int ravel_em_seg_sum_bwd(const void* write_addr, const void* read_addr, int addr
  *                     stream of grad_sum[r].
  * Addresses, mask and k are the forward's.  grad_values [B,T,C,k,D] or
  * grad_sum [B,T,C,D] may be NULL (no gradient).  Needs no sources.
- * Deterministic; one rounding of the total.  Takes k <= 8, T <= 2^23 and
+ * Deterministic; one rounding of the total.  Takes k <= 8, T <= 2^24 and
  * gradient rows of one batch row below 2^31 bytes (RAVEL_EM_EINVAL, and a
  * workspace query of 0, otherwise); any D.  The workspace carries the status
  * word as the sorting calls' do.

@@ -460,6 +460,85 @@ size_t latest_k_ws_t(const Tape& tp, int64_t k, bool link, bool want_src) {
   return bp.off;
 }
 
+// ------------------------------------------------------- tape walks --
+// Backward of the segmented sum, of the latest-k lookup or of both of one tape
+// in one segmented walk (em_walk.h): reads = writes without a mask walk the
+// tape's own sorted keys, others the sorted tape of reads and writes together.
+// Which of the two, from the call's address arguments.
+struct TapeArgs {
+  AddrIn w, r;
+  bool has_read = false;
+  const uint8_t* wmask = nullptr;
+  bool merged = false;  // w is a merged tape already (RAVEL_EM_TAPE)
+  bool same() const { return !has_read && !wmask && !merged; }
+};
+
+Tape walk_tape(const Tape& tp, bool same) { return same ? tp : merged_tape(tp); }
+
+size_t tape_walk_ws(const Tape& tp, int64_t D, int dtype, int64_t k, bool same) {
+  const Tape wt = walk_tape(tp, same);
+  Bump bp(nullptr);
+  if (wt.wide())
+    take_sort<uint64_t>(bp, wt);
+  else
+    take_sort<uint32_t>(bp, wt);
+  bp.take<uint64_t>(walk_words(tp.nseg(), wt.T, D, dtype, k));
+  return bp.off;
+}
+
+template <typename U>
+int tape_walk_run(const TapeArgs& ta, const Tape& tape, int64_t D, int dtype, bool fwd,
+                  const void* sum_in, const void* val_in, int64_t k, void* out, uint8_t* omask,
+                  void* val_out, uint8_t* vmask, void* ws, size_t wsb, hipStream_t s) {
+  const bool same = ta.same();
+  Tape tp = tape;
+  Tape wt = walk_tape(tp, same);
+  Bump bp(ws);
+  SortWs<U> sw = take_sort<U>(bp, wt);
+  tp.status = wt.status = sw.status;
+  const size_t nw = walk_words(tp.nseg(), wt.T, D, dtype, k);
+  uint64_t* words = bp.take<uint64_t>(nw);
+  if (int rc = check_ws(bp, wsb)) return rc;
+  AddrIn in = ta.w;
+  hipError_t e = hipSuccess;
+  if (ta.merged) {
+    in.kind = merged_kind(tp.A);
+  } else if (!same) {
+    // produced addresses decode into the key buffer that the key build fills
+    // last; the merged tape goes into the other, which its first pass overwrites
+    AddrIn wd, rd;
+    const size_t half = (size_t)tp.n() * sizeof(U);
+    e = compact_addresses(ta.w, tp, sw.ka, &wd, s);
+    rd = wd;
+    if (e == hipSuccess && ta.has_read)
+      e = compact_addresses(ta.r, tp, (char*)sw.ka + half, &rd, s);
+    if (e == hipSuccess) e = merge_addresses(wd, rd, ta.wmask, tp, sw.kb, &in, s);
+    if (e != hipSuccess) return hip_fail(e, "merged tape");
+  }
+  U* sorted = nullptr;
+  stage_begin(kStageSort, s);
+  e = sort_call<U>(in, nullptr, wt, sw, &sorted, s, nw ? (uint32_t*)words : nullptr,
+                   2 * (int64_t)nw);
+  stage_end(kStageSort, s);
+  if (e != hipSuccess) return hip_fail(e, "sort");
+  stage_begin(kStageSum, s);
+  e = tape_walk(sorted, sizeof(U) == 8, wt.tbits, same, fwd, tp, D, dtype, sum_in, val_in, k, out,
+                omask, val_out, vmask, words, s);
+  stage_end(kStageSum, s);
+  if (e != hipSuccess) return hip_fail(e, "segmented walk");
+  return RAVEL_EM_OK;
+}
+
+int tape_walk_call(const TapeArgs& ta, const Tape& tp, int64_t D, int dtype, bool fwd,
+                   const void* sum_in, const void* val_in, int64_t k, void* out, uint8_t* omask,
+                   void* val_out, uint8_t* vmask, void* ws, size_t wsb, hipStream_t s) {
+  return walk_tape(tp, ta.same()).wide()
+             ? tape_walk_run<uint64_t>(ta, tp, D, dtype, fwd, sum_in, val_in, k, out, omask,
+                                       val_out, vmask, ws, wsb, s)
+             : tape_walk_run<uint32_t>(ta, tp, D, dtype, fwd, sum_in, val_in, k, out, omask,
+                                       val_out, vmask, ws, wsb, s);
+}
+
 // ---------------------------------------------------------- seg-sum --
 
 template <typename U>
@@ -497,6 +576,31 @@ SumWs<U> take_sum(Bump& bp, const Tape& tp, int64_t D, int dtype, bool direct, b
 }
 
 template <typename U>
+size_t sum_ws_t(const Tape& tp, int64_t D, int dtype, bool direct, bool backward) {
+  Bump bp(nullptr);
+  take_sum<U>(bp, tp, D, dtype, direct, backward);
+  return bp.off;
+}
+
+// Workspace of a forward sum: the form depends on the pointers' alignment, so
+// room for any of them.
+size_t seg_sum_ws(const Tape& tp, int64_t D, int dtype, bool direct) {
+  const size_t a = tp.wide() ? sum_ws_t<uint64_t>(tp, D, dtype, direct, false)
+                             : sum_ws_t<uint32_t>(tp, D, dtype, direct, false);
+  const size_t b = walk_applies(tp, D, dtype, 0) ? tape_walk_ws(tp, D, dtype, 0, direct) : 0;
+  return a > b ? a : b;
+}
+
+TapeArgs tape_args(const AddrIn& wa, const AddrIn* ra, const uint8_t* wmask) {
+  TapeArgs ta;
+  ta.w = wa;
+  if (ra) ta.r = *ra;
+  ta.has_read = ra != nullptr;
+  ta.wmask = wmask;
+  return ta;
+}
+
+template <typename U>
 int seg_sum_run(const AddrIn& wa, const AddrIn* ra, const uint8_t* wmask,
                 const void* payload, int dtype, const Tape& tape, int64_t D, void* out_sum,
                 uint8_t* out_mask, void* ws, size_t wsb, hipStream_t s) {
@@ -505,7 +609,9 @@ int seg_sum_run(const AddrIn& wa, const AddrIn* ra, const uint8_t* wmask,
   Tape tp = tape;
   SumWs<U> w = take_sum<U>(bp, tp, D, dtype, direct, false);
   tp.status = w.sw.status;
-  if (int rc = check_ws(bp, wsb)) return rc;
+  if (wsb < seg_sum_ws(tp, D, dtype, direct))
+    return fail(RAVEL_EM_EWORKSPACE, "workspace of %zu bytes, need %zu", wsb,
+                seg_sum_ws(tp, D, dtype, direct));
   if (seg_sum_merged_applies(tp, D, dtype, payload, out_sum)) {
     // short tapes: one block per segment, reads and writes merged in LDS
     stage_begin(kStageSum, s);
@@ -518,6 +624,9 @@ int seg_sum_run(const AddrIn& wa, const AddrIn* ra, const uint8_t* wmask,
     if (e != hipSuccess) return hip_fail(e, "segmented sum");
     return RAVEL_EM_OK;
   }
+  if (walk_applies(tp, D, dtype, 0))
+    return tape_walk_call(tape_args(wa, ra, wmask), tp, D, dtype, true, payload, nullptr, 0,
+                          out_sum, out_mask, nullptr, nullptr, ws, wsb, s);
   U* sorted = nullptr;
   stage_begin(kStageSort, s);
   hipError_t e = sort_call<U>(wa, wmask, tp, w.sw, &sorted, s, (uint32_t*)w.walk,
@@ -566,99 +675,13 @@ int seg_sum_bwd_run(const AddrIn& wa, const AddrIn* ra, const uint8_t* wmask,
   return RAVEL_EM_OK;
 }
 
-// ------------------------------------------------------- tape walks --
-// Backward of the segmented sum, of the latest-k lookup or of both of one tape
-// in one segmented walk (em_walk.h): reads = writes without a mask walk the
-// tape's own sorted keys, others the sorted tape of reads and writes together.
-// Which of the two, from the call's address arguments.
-struct TapeArgs {
-  AddrIn w, r;
-  bool has_read = false;
-  const uint8_t* wmask = nullptr;
-  bool merged = false;  // w is a merged tape already (RAVEL_EM_TAPE)
-  bool same() const { return !has_read && !wmask && !merged; }
-};
-
-Tape walk_tape(const Tape& tp, bool same) { return same ? tp : merged_tape(tp); }
-
-size_t tape_walk_ws(const Tape& tp, int64_t D, int dtype, int64_t k, bool same) {
-  const Tape wt = walk_tape(tp, same);
-  Bump bp(nullptr);
-  if (wt.wide())
-    take_sort<uint64_t>(bp, wt);
-  else
-    take_sort<uint32_t>(bp, wt);
-  bp.take<uint64_t>(walk_words(tp.nseg(), wt.T, D, dtype, k));
-  return bp.off;
-}
-
-template <typename U>
-int tape_walk_run(const TapeArgs& ta, const Tape& tape, int64_t D, int dtype, bool fwd,
-                  const void* sum_in, const void* val_in, int64_t k, void* out, uint8_t* omask,
-                  void* ws, size_t wsb, hipStream_t s) {
-  const bool same = ta.same();
-  Tape tp = tape;
-  Tape wt = walk_tape(tp, same);
-  Bump bp(ws);
-  SortWs<U> sw = take_sort<U>(bp, wt);
-  tp.status = wt.status = sw.status;
-  const size_t nw = walk_words(tp.nseg(), wt.T, D, dtype, k);
-  uint64_t* words = bp.take<uint64_t>(nw);
-  if (int rc = check_ws(bp, wsb)) return rc;
-  AddrIn in = ta.w;
-  hipError_t e = hipSuccess;
-  if (ta.merged) {
-    in.kind = merged_kind(tp.A);
-  } else if (!same) {
-    // produced addresses decode into the key buffer that the key build fills
-    // last; the merged tape goes into the other, which its first pass overwrites
-    AddrIn wd, rd;
-    const size_t half = (size_t)tp.n() * sizeof(U);
-    e = compact_addresses(ta.w, tp, sw.ka, &wd, s);
-    rd = wd;
-    if (e == hipSuccess && ta.has_read)
-      e = compact_addresses(ta.r, tp, (char*)sw.ka + half, &rd, s);
-    if (e == hipSuccess) e = merge_addresses(wd, rd, ta.wmask, tp, sw.kb, &in, s);
-    if (e != hipSuccess) return hip_fail(e, "merged tape");
-  }
-  U* sorted = nullptr;
-  stage_begin(kStageSort, s);
-  e = sort_call<U>(in, nullptr, wt, sw, &sorted, s, nw ? (uint32_t*)words : nullptr,
-                   2 * (int64_t)nw);
-  stage_end(kStageSort, s);
-  if (e != hipSuccess) return hip_fail(e, "sort");
-  stage_begin(kStageSum, s);
-  e = tape_walk(sorted, sizeof(U) == 8, wt.tbits, same, fwd, tp, D, dtype, sum_in, val_in, k, out,
-                omask, words, s);
-  stage_end(kStageSum, s);
-  if (e != hipSuccess) return hip_fail(e, "segmented walk");
-  return RAVEL_EM_OK;
-}
-
-int tape_walk_call(const TapeArgs& ta, const Tape& tp, int64_t D, int dtype, bool fwd,
-                   const void* sum_in, const void* val_in, int64_t k, void* out, uint8_t* omask,
-                   void* ws, size_t wsb, hipStream_t s) {
-  return walk_tape(tp, ta.same()).wide()
-             ? tape_walk_run<uint64_t>(ta, tp, D, dtype, fwd, sum_in, val_in, k, out, omask, ws,
-                                       wsb, s)
-             : tape_walk_run<uint32_t>(ta, tp, D, dtype, fwd, sum_in, val_in, k, out, omask, ws,
-                                       wsb, s);
-}
-
-template <typename U>
-size_t sum_ws_t(const Tape& tp, int64_t D, int dtype, bool direct, bool backward) {
-  Bump bp(nullptr);
-  take_sum<U>(bp, tp, D, dtype, direct, backward);
-  return bp.off;
-}
-
 // ----------------------------------------------- latest-k and sum --
 // The latest-k lookup and the segmented sum of one tape (the pair of calls of
 // ravel_lm/model.py:366-386) over one sort:
 //   short tapes: the merged sum kernel, whose LDS sort already orders reads
 //     and writes, also writes every read's latest-k rows (one launch);
-//   long tapes, reads = writes, k = 1: one full sort, then the walker's sum
-//     walk also stores each record's predecessor row (the latest-1 value);
+//   others up to k = 8: one sort of the tape (reads and writes together unless
+//     they share their addresses), then one segmented walk;
 //   otherwise: the two operators one after the other on the same workspace,
 //     their status words ORed.
 __global__ void status_keep_kernel(uint32_t* __restrict__ hdr, int restore) {
@@ -694,22 +717,19 @@ int latest_k_sum_run(const AddrIn& wa, const AddrIn* ra, const uint8_t* wmask,
     if (e != hipSuccess) return hip_fail(e, "segmented sum and latest-k");
     return RAVEL_EM_OK;
   }
-  if (!ra && !wmask && k == 1 && seg_sum_joint_applies(tp, D, dtype, payload, out_sum, out_values)) {
-    Bump bp(ws);
-    SumWs<U> w = take_sum<U>(bp, tp, D, dtype, true, false);
-    tp.status = w.sw.status;
-    if (int rc = check_ws(bp, wsb)) return rc;
-    U* sorted = nullptr;
-    stage_begin(kStageSort, s);
-    hipError_t e = sort_call<U>(wa, nullptr, tp, w.sw, &sorted, s, (uint32_t*)w.walk,
-                                2 * w.walk_words);
-    stage_end(kStageSort, s);
-    if (e != hipSuccess) return hip_fail(e, "sort");
-    stage_begin(kStageSum, s);
-    e = seg_sum_joint<U>(sorted, payload, dtype, tp, D, out_sum, out_sum_mask, out_values,
-                         out_mask, out_src, w.walk, s);
-    stage_end(kStageSum, s);
-    if (e != hipSuccess) return hip_fail(e, "segmented sum and latest-1");
+  if (walk_applies(tp, D, dtype, k)) {
+    int rc = tape_walk_call(tape_args(wa, ra, wmask), tp, D, dtype, true, payload, nullptr, k,
+                            out_sum, out_sum_mask, out_values, out_mask, ws, wsb, s);
+    if (rc != RAVEL_EM_OK || !out_src) return rc;
+    // the walk keeps no sources: a caller that wants them has them resolved too
+    status_keep_kernel<<<1, 64, 0, s>>>((uint32_t*)ws, 0);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e, "status word");
+    rc = resolve_run<U>(wa, ra, wmask, tape, k, out_src, ws, wsb, s);
+    if (rc != RAVEL_EM_OK) return rc;
+    status_keep_kernel<<<1, 64, 0, s>>>((uint32_t*)ws, 1);
+    e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e, "status word");
     return RAVEL_EM_OK;
   }
   if (int rc = latest_k_run<U>(wa, ra, wmask, payload, row_bytes, tape, k, out_values, out_mask,
@@ -731,8 +751,9 @@ template <typename U>
 size_t latest_k_sum_ws_t(const Tape& tp, int64_t D, int dtype, int64_t k, bool link,
                          bool want_src) {
   const size_t a = latest_k_ws_t<U>(tp, k, link, want_src);
-  const size_t b = sum_ws_t<U>(tp, D, dtype, link, false);
-  return a > b ? a : b;
+  const size_t b = seg_sum_ws(tp, D, dtype, link);
+  const size_t c = walk_applies(tp, D, dtype, k) ? tape_walk_ws(tp, D, dtype, k, link) : 0;
+  return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
 // ------------------------------------------- static scratch (no allocation) --
@@ -1409,8 +1430,7 @@ size_t ravel_em_seg_sum_workspace(int64_t B, int64_t T, int64_t C, int64_t D, in
   const int64_t rows = split_rows(B, T * C);
   const Tape tp = make_tape(B < rows ? B : rows, T, C, A, has_mask != 0, kWrap);
   const bool direct = !has_read && !has_mask;
-  return tp.wide() ? sum_ws_t<uint64_t>(tp, D, payload_dtype, direct, false)
-                   : sum_ws_t<uint32_t>(tp, D, payload_dtype, direct, false);
+  return seg_sum_ws(tp, D, payload_dtype, direct);
 }
 
 int ravel_em_seg_sum_fwd(const void* write_addr, const void* read_addr, int addr_dtype,
@@ -1491,13 +1511,8 @@ int ravel_em_seg_sum_bwd(const void* write_addr, const void* read_addr, int addr
     const void* g = at(grad_sum, r0 * row_bytes);
     void* gp = at(grad_payload, r0 * row_bytes);
     if (walk_applies(t, D, payload_dtype, 0)) {
-      TapeArgs ta;
-      ta.w = w;
-      ta.r = r;
-      ta.has_read = rp != nullptr;
-      ta.wmask = wm;
-      return tape_walk_call(ta, t, D, payload_dtype, false, g, nullptr, 0, gp, nullptr, workspace,
-                            workspace_bytes, s);
+      return tape_walk_call(tape_args(w, rp, wm), t, D, payload_dtype, false, g, nullptr, 0, gp, nullptr, nullptr,
+                            nullptr, workspace, workspace_bytes, s);
     }
     return t.wide() ? seg_sum_bwd_run<uint64_t>(w, rp, wm, g, payload_dtype, t, D, gp, workspace,
                                                 workspace_bytes, s)
@@ -1574,7 +1589,7 @@ int ravel_em_latest_k_sum_bwd(const void* write_addr, const void* read_addr, int
   most.B = B < rows ? B : rows;
   if (!walk_applies(most, D, payload_dtype, k))
     return fail(RAVEL_EM_EINVAL,
-                "the joint backward takes k <= 8, T <= 2^23 and T*C*k*D elements of one batch "
+                "the joint backward takes k <= 8, T <= 2^24 and T*C*k*D elements of one batch "
                 "row below 2^31 bytes (T=%lld C=%lld D=%lld k=%lld)",
                 (long long)T, (long long)C, (long long)D, (long long)k);
   return split_batch(B, rows, workspace, workspace_bytes, s, [&](int64_t nb, int64_t b0) -> int {
@@ -1593,7 +1608,7 @@ int ravel_em_latest_k_sum_bwd(const void* write_addr, const void* read_addr, int
     }
     return tape_walk_call(ta, t, D, payload_dtype, false, at(grad_sum, r0 * row_bytes),
                           at(grad_values, r0 * k * row_bytes), k, at(grad_payload, r0 * row_bytes),
-                          nullptr, workspace, workspace_bytes, s);
+                          nullptr, nullptr, nullptr, workspace, workspace_bytes, s);
   });
 }
 

@@ -320,17 +320,6 @@ hipError_t seg_sum_merged(const AddrIn& wa, const AddrIn* ra, const uint8_t* wma
                           const void* payload, int dtype, const Tape& tp, int64_t D, void* out,
                           uint8_t* omask, hipStream_t s, int64_t k = 0, void* vout = nullptr,
                           uint8_t* vmask = nullptr, int32_t* osrc = nullptr);
-// Forward sums and latest-1 lookup of reads = writes over one sorted tape in
-// one walker launch (seg_sum_joint_applies: rows of 1..64 16-byte units, a
-// power of two; 16-byte aligned rows): out_sum/omask as seg_sum's direct form,
-// out_values [B,T,C,1,D] and vmask [B,T,C,1] as the latest-1 lookup, vsrc
-// (optional) its int32 sources.  Same workspace as seg_sum.
-bool seg_sum_joint_applies(const Tape& tp, int64_t D, int dtype, const void* payload,
-                           const void* out_sum, const void* out_values);
-template <typename U>
-hipError_t seg_sum_joint(const U* sorted, const void* payload, int dtype, const Tape& tp,
-                         int64_t D, void* out_sum, uint8_t* omask, void* out_values,
-                         uint8_t* vmask, int32_t* vsrc, uint64_t* walk, hipStream_t s);
 size_t seg_sum_chunks(const Tape& tp);
 size_t acc_bytes(int dtype);
 size_t seg_sum_walk_words(const Tape& tp, int64_t D, int dtype);
@@ -355,14 +344,16 @@ hipError_t seg_sum_bwd(const U* sorted, const int32_t* spos, const void* grad_ou
 
 // Segmented walk of a sorted tape (em_walk.h): fwd false, the backward (out =
 // per-write gradient from sum_in [B,T,C,D] and / or val_in [B,T,C,k,D]); fwd true,
-// the forward sum (out, omask from sum_in = payload).  keys: same (reads at the
+// the forward sum (out, omask from sum_in = payload) and, with val_out, the
+// latest-k values and mask (val_out [B,T,C,k,D], vmask [B,T,C,k]).  keys: same (reads at the
 // write addresses, no mask) the tape's sorted keys, else those of
 // merged_tape(tp), tbits its tape's; words: walk_words() words, zero on entry.
 bool walk_applies(const Tape& tp, int64_t D, int dtype, int64_t k);
 size_t walk_words(int64_t nseg, int64_t L, int64_t D, int dtype, int64_t k);
 hipError_t tape_walk(const void* keys, bool wide, int tbits, bool same, bool fwd, const Tape& tp,
                      int64_t D, int dtype, const void* sum_in, const void* val_in, int64_t k,
-                     void* out, uint8_t* omask, uint64_t* words, hipStream_t s);
+                     void* out, uint8_t* omask, void* val_out, uint8_t* vmask, uint64_t* words,
+                     hipStream_t s);
 // Reads and writes of a tape as one address tensor [B,2T,C] (even steps the
 // reads, odd the writes, a masked write the address A) in buf (merged_bytes()),
 // and the tape that sorts it.  wa and ra are dense inputs of one kind.

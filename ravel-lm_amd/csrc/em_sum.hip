@@ -274,7 +274,6 @@ size_t seg_sum_status_words(const Tape& tp, int64_t D, size_t acc_size) {
 // blocks already claimed.
 constexpr int kWalkThreads = 256;
 constexpr int kWalkBatch = 16;
-constexpr int kFastBatch = 16;  // items a lane has in flight in the branch-free walks
 // Branch-free walks through buffer descriptors: a 32-bit code word per item
 // (the time in bits 0..23, flags above) and byte offsets below 2^30, so an
 // offset with bit 30 or 31 set lies past every range: the buffer unit turns
@@ -326,21 +325,13 @@ __device__ __forceinline__ void add_unit(Acc* acc, u32x4 x) {
   for (int j = 0; j < CPU; ++j) acc[j] += LoadF::load(cv.e[j]);
 }
 
-// VAL (the fast form, reads = writes): the final walk also writes every
-// record's latest-1 value, the row of the position before it in its run (the
-// row the walk has just added; +0.0 at a run start), into vout at the sum's
-// offset, with vmask the same mask byte into vmask and, with vsrc, that row's
-// record id (-1 at a run start): the latest-1 lookup of the same sorted tape
-// with no sort, link or gather of its own.
 template <typename U, typename XIn, typename XOut, typename Acc, typename LoadF, typename StoreF,
-          bool REV, bool IN_SORTED, bool INCL, bool OUT_SORTED, bool WMASK, bool RT, bool FAST,
-          bool VAL = false>
+          bool REV, bool IN_SORTED, bool INCL, bool OUT_SORTED, bool WMASK, bool RT>
 __global__ __launch_bounds__(kWalkThreads) void segsum_walk_kernel(
     const U* __restrict__ sorted, const XIn* __restrict__ in, int64_t T, int64_t C, int64_t D,
     int tbits, int G, int64_t nparts, XOut* __restrict__ out, uint8_t* __restrict__ omask,
     uint64_t* __restrict__ status, uint64_t* __restrict__ tickets, uint32_t* __restrict__ err,
-    int64_t nout, XOut* __restrict__ vout = nullptr, uint8_t* __restrict__ vmask = nullptr,
-    int32_t* __restrict__ vsrc = nullptr) {
+    int64_t nout) {
   constexpr int CPU = 16 / (int)sizeof(XIn);  // columns per lane
   using OutV = typename Unit<CPU * (int)sizeof(XOut)>::T;
   constexpr int NWMAX = kWalkThreads;  // walkers when G == 1
@@ -350,12 +341,6 @@ __global__ __launch_bounds__(kWalkThreads) void segsum_walk_kernel(
   __shared__ Acc tl[kWalkThreads * CPU];  // [walker][column]
   __shared__ uint32_t s_part;
   __shared__ uint8_t s_next;  // the position after the part starts a run (or the segment ends)
-  // FAST (forward exclusive sums by record, rows at 32-bit offsets of the
-  // segment's base): one code word per position, walks without branches
-  static_assert(!FAST || (!REV && !IN_SORTED && !INCL && !OUT_SORTED && !RT), "fast form");
-  static_assert(!VAL || (FAST && WMASK), "values ride on the fast form");
-  __shared__ __align__(16) uint32_t cw[FAST ? kPartPos : 4];
-  __shared__ uint32_t s_ptime;  // VAL: time of the position before the part
   // Exclusive forward sums never add the last row of a run to any output:
   // those rows are not loaded (on a uniform tape most runs are one record).
   constexpr bool SKIP_LAST = !INCL && !REV;
@@ -384,11 +369,9 @@ __global__ __launch_bounds__(kWalkThreads) void segsum_walk_kernel(
       start = (kk[i] >> tbits) != (kk[i - 1] >> tbits);
     } else if (wi == 0) {
       start = true;
-      if (VAL) s_ptime = 0u;
     } else {
       const U prev = sk[REV ? (T - wi) : (wi - 1)];
       start = (kk[0] >> tbits) != (prev >> tbits);
-      if (VAL) s_ptime = (uint32_t)(prev & tmask);
     }
     st[i] = start ? 1 : 0;
   }
@@ -402,19 +385,9 @@ __global__ __launch_bounds__(kWalkThreads) void segsum_walk_kernel(
   };
   const int NW = kWalkThreads / G;
   const int w = tid / G, v = tid - (tid / G) * G;
-  // FAST: positions [n, nr) pad the walkers' ranges to whole batches
-  const int nr = FAST ? (n + kFastBatch - 1) & ~(kFastBatch - 1) : n;
-  if constexpr (FAST) {
-    for (int i = tid; i < nr; i += kWalkThreads)
-      cw[i] = i < n ? ((uint32_t)(kk[i] & tmask) | (st[i] ? kCodeStart : 0u) |
-                       (needed(i) ? 0u : kCodeNoLoad))
-                    : (kCodeNoLoad | kCodeNoStore);
-    __syncthreads();
-  }
-  const int len = FAST ? ((((nr + NW - 1) / NW) + kFastBatch - 1) & ~(kFastBatch - 1))
-                       : (n + NW - 1) / NW;
-  const int rs = w * len < nr ? w * len : nr;
-  const int re = (rs + len) < nr ? (rs + len) : nr;
+  const int len = (n + NW - 1) / NW;
+  const int rs = w * len < n ? w * len : n;
+  const int re = (rs + len) < n ? (rs + len) : n;
   // Row indices fit in 32 bits (N < 2^31): record (b*T + t)*C + c, or the
   // sorted position segbase + pos.
   const int32_t vbase = (int32_t)((b * T) * C + c), Ci = (int32_t)C;
@@ -424,79 +397,18 @@ __global__ __launch_bounds__(kWalkThreads) void segsum_walk_kernel(
   auto irow = [&](int i) -> int32_t { return IN_SORTED ? sp_of(i) : rec_of(i); };
   auto orow = [&](int i) -> int32_t { return OUT_SORTED ? sp_of(i) : rec_of(i); };
   const u32x4* inv = (const u32x4*)in;
-  // FAST: the segment's rows through buffer descriptors (row t's unit v at
-  // byte t * tstride + 16 v of the segment's base, in the payload and the
-  // output alike); the code word's bits 29..31 are flags above the time, which
-  // the 24-bit multiply ignores.
-  const uint32_t tstride = (uint32_t)(C * G * 16), v16 = (uint32_t)v * 16u;
-  const int ext = FAST ? (int)(T * C * G * 16) : 0;  // below 2^30 in the fast form
-  const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)((const unsigned char*)in + (int64_t)vbase * G * 16), 0, ext, kRsrcWord3);
-  const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)((unsigned char*)out + (int64_t)vbase * G * 16), 0, ext, kRsrcWord3);
   Acc acc[CPU];
-  // VAL: the row of the item before the next one (zeros where not loaded)
-  u32x4 vprev = {0u, 0u, 0u, 0u};
-  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(VAL ? (unsigned char*)vout + (int64_t)vbase * G * 16 : (unsigned char*)vout), 0,
-      VAL ? ext : 0, kRsrcWord3);
-  // Items [from, to) in whole batches from the one holding `from` (items
-  // outside are pads): a run start resets the sum, every position stores the
-  // sum before its own row (STORE), every needed row is added.
-  auto walk_fast = [&](int from, int to, auto store_tag) {
-    constexpr bool STORE = decltype(store_tag)::value;
-    constexpr int aux = STORE ? kBufNontemporal : 0;
-    constexpr uint32_t kPad = kCodeNoLoad | kCodeNoStore;
-    if constexpr (FAST)
-    for (int i0 = from & ~(kFastBatch - 1); i0 < to; i0 += kFastBatch) {
-      uint32_t c4w[kFastBatch];
-#pragma unroll
-      for (int q4 = 0; q4 < kFastBatch / 4; ++q4) {
-        const u32x4 c4 = *(const u32x4*)&cw[i0 + 4 * q4];
-        c4w[4 * q4] = c4.x, c4w[4 * q4 + 1] = c4.y, c4w[4 * q4 + 2] = c4.z, c4w[4 * q4 + 3] = c4.w;
-      }
-#pragma unroll
-      for (int m = 0; m < kFastBatch; ++m)
-        if (i0 + m < from || i0 + m >= to) c4w[m] = kPad;
-      u32x4 x[kFastBatch];
-#pragma unroll
-      for (int m = 0; m < kFastBatch; ++m)
-        x[m] = __builtin_amdgcn_raw_buffer_load_b128(
-            prs, (__umul24(c4w[m], tstride) + v16) | (c4w[m] & kCodeNoLoad), 0, aux);
-#pragma unroll
-      for (int m = 0; m < kFastBatch; ++m) {
-        const uint32_t k = c4w[m];
-        const bool stt = k & kCodeStart;
-#pragma unroll
-        for (int j = 0; j < CPU; ++j) acc[j] = stt ? Acc(0) : acc[j];
-        if (STORE)
-          __builtin_amdgcn_raw_buffer_store_b128(pack_unit<XOut, StoreF, Acc, CPU>(acc), ors,
-                                                 (__umul24(k, tstride) + v16) | (k & kCodeNoStore), 0,
-                                                 aux);
-        if (STORE && VAL) {
-          const u32x4 z = {0u, 0u, 0u, 0u};
-          __builtin_amdgcn_raw_buffer_store_b128(stt ? z : vprev, vrs,
-                                                 (__umul24(k, tstride) + v16) | (k & kCodeNoStore), 0,
-                                                 aux);
-          vprev = x[m];
-        }
-        add_unit<XIn, LoadF, Acc, CPU>(acc, x[m]);  // zeros where not loaded
-      }
-    }
-  };
   // 2. tail of the walker's range
   int last = -1;
   for (int i = rs + v; i < re; i += G)
-    if (FAST ? (cw[i] & kCodeStart) != 0 : st[i] != 0) last = i;
+    if (st[i] != 0) last = i;
   for (int o = 1; o < G; o <<= 1) {
     const int other = __shfl_xor(last, o, kWave);
     last = other > last ? other : last;
   }
 #pragma unroll
   for (int j = 0; j < CPU; ++j) acc[j] = Acc(0);
-  if constexpr (FAST) {
-    walk_fast(last >= 0 ? last : rs, re, std::false_type{});
-  } else {
+  {
     for (int i0 = (last >= 0 ? last : rs); i0 < re; i0 += kWalkBatch) {
       u32x4 x[kWalkBatch];
 #pragma unroll
@@ -576,44 +488,6 @@ __global__ __launch_bounds__(kWalkThreads) void segsum_walk_kernel(
   // non-temporal and leave L2 to the keys.
 #pragma unroll
   for (int j = 0; j < CPU; ++j) acc[j] = tl[w * ncol + v * CPU + j];
-  if constexpr (FAST) {
-    if constexpr (VAL) {
-      // the row before the range's first item, when that item continues a run
-      if (rs < re) {
-        const uint32_t pc = rs > 0 ? cw[rs - 1] : s_ptime;
-        const bool cont = (cw[rs] & kCodeStart) == 0;  // false at p0 == 0
-        vprev = __builtin_amdgcn_raw_buffer_load_b128(
-            prs, (__umul24(pc, tstride) + v16) | (cont ? 0u : kCodeNoLoad), 0, kBufNontemporal);
-      }
-    }
-    walk_fast(rs, re, std::true_type{});
-    if (WMASK) {  // a record's mask: some earlier record of its run (byte stores after the walk)
-      __syncthreads();
-      const __amdgpu_buffer_rsrc_t mrs =
-          __builtin_amdgcn_make_buffer_rsrc((void*)(omask + vbase), 0, (int)(T * C), kRsrcWord3);
-      const __amdgpu_buffer_rsrc_t vmrs = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(VAL && vmask ? vmask + vbase : vmask), 0, VAL && vmask ? (int)(T * C) : 0,
-          kRsrcWord3);
-      const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(VAL && vsrc ? vsrc + vbase : vsrc), 0, VAL && vsrc ? (int)(T * C * 4) : 0,
-          kRsrcWord3);
-      for (int i = tid; i < n; i += kWalkThreads) {
-        const uint32_t k = cw[i];
-        const uint8_t has = (k & kCodeStart) ? 0 : 1;
-        const uint32_t moff = (k & kCodeTime) * (uint32_t)C;
-        __builtin_amdgcn_raw_buffer_store_b8(has, mrs, moff, 0, 0);
-        if (VAL) {
-          if (vmask) __builtin_amdgcn_raw_buffer_store_b8(has, vmrs, moff, 0, 0);
-          if (vsrc) {
-            const uint32_t pt = i > 0 ? (cw[i - 1] & kCodeTime) : s_ptime;
-            const int32_t sr = has ? vbase + (int32_t)pt * Ci : -1;
-            __builtin_amdgcn_raw_buffer_store_b32((uint32_t)sr, srs, moff * 4u, 0, 0);
-          }
-        }
-      }
-    }
-    return;
-  }
   for (int i0 = rs; i0 < re; i0 += kWalkBatch) {
     u32x4 x[kWalkBatch];
 #pragma unroll
@@ -1428,26 +1302,10 @@ hipError_t run_segsum(const U* sorted, const XIn* in, const Tape& tp, int64_t D,
     const int64_t blocks = tp.nseg() * nparts;
     if (blocks > INT32_MAX) return hipErrorInvalidValue;
     uint64_t* tickets = walk + seg_sum_status_words(tp, D, sizeof(Acc));
-    // the branch-free form: forward exclusive sums by record whose rows sit at
-    // offsets below 2^30 of their segment's base (24-bit time and stride)
-    constexpr bool kFastForm = !REV && !IN_SORTED && !INCL && !OUT_SORTED && !RT &&
-                               std::is_same<XIn, XOut>::value;
-    const bool fast = kFastForm && tp.T <= ((int64_t)1 << 24) &&
-                      tp.C * in_bytes < ((int64_t)1 << 24) &&
-                      tp.T * tp.C * in_bytes <= ((int64_t)1 << 30);
-#define REM_WALK(F)                                                                              \
-  segsum_walk_kernel<U, XIn, XOut, Acc, LoadF, StoreF, REV, IN_SORTED, INCL, OUT_SORTED, WMASK, RT, \
-                     F><<<(unsigned)blocks, kWalkThreads, 0, s>>>(                                \
-      sorted, in, tp.T, tp.C, D, tp.tbits, (int)G, nparts, out, omask, walk, tickets, tp.status, nout)
-    if constexpr (kFastForm) {
-      if (fast)
-        REM_WALK(true);
-      else
-        REM_WALK(false);
-    } else {
-      REM_WALK(false);
-    }
-#undef REM_WALK
+    segsum_walk_kernel<U, XIn, XOut, Acc, LoadF, StoreF, REV, IN_SORTED, INCL, OUT_SORTED, WMASK, RT>
+        <<<(unsigned)blocks, kWalkThreads, 0, s>>>(sorted, in, tp.T, tp.C, D, tp.tbits, (int)G,
+                                                   nparts, out, omask, walk, tickets, tp.status,
+                                                   nout);
     return hipGetLastError();
   }
   const int64_t nch_seg = (tp.T + kChunk - 1) / kChunk;
@@ -1520,44 +1378,6 @@ hipError_t seg_sum_bwd_t(const U* sorted, const int32_t* spos, const void* grad_
       sorted, (const G*)gacc, tp, D, (S*)grad_payload, nullptr, (Acc*)tail, flag, (Acc*)carry, walk, s);
 }
 
-// Forward sums and latest-1 values of reads = writes in one walk (the fast
-// walker form with VAL).
-bool joint_walk_applies(const Tape& tp, int64_t row_bytes, const void* payload, const void* out,
-                        const void* vout) {
-  const int64_t G = row_bytes / 16;
-  return row_bytes % 16 == 0 && G >= 1 && G <= 64 && (G & (G - 1)) == 0 &&
-         (((uintptr_t)payload | (uintptr_t)out | (uintptr_t)vout) & 15) == 0 &&
-         tp.T <= ((int64_t)1 << 24) && tp.C * row_bytes < ((int64_t)1 << 24) &&
-         tp.T * tp.C * row_bytes <= ((int64_t)1 << 30) &&
-         tp.nseg() * ((tp.T + kPartPos - 1) / kPartPos) <= INT32_MAX;
-}
-
-template <int DT, typename U>
-hipError_t seg_sum_joint_t(const U* sorted, const void* payload, const Tape& tp, int64_t D,
-                           void* out_sum, uint8_t* omask, void* out_values, uint8_t* vmask,
-                           int32_t* vsrc, uint64_t* walk, hipStream_t s) {
-  using E = Elem<DT>;
-  using S = typename E::store_t;
-  using Acc = typename E::acc_t;
-  const int64_t row_bytes = D * (int64_t)sizeof(S);
-  if (!tp.status || !walk || !joint_walk_applies(tp, row_bytes, payload, out_sum, out_values))
-    return hipErrorInvalidValue;
-  const int64_t G = row_bytes / 16;
-  const int64_t nparts = (tp.T + kPartPos - 1) / kPartPos;
-  const int64_t blocks = tp.nseg() * nparts;
-  uint64_t* tickets = walk + seg_sum_status_words(tp, D, sizeof(Acc));
-  // The two masks of latest-1 are the same bytes: the walk stores them once,
-  // at random records, and one sequential copy makes the other.
-  segsum_walk_kernel<U, S, S, Acc, E, E, false, false, false, false, true, false, true, true>
-      <<<(unsigned)blocks, kWalkThreads, 0, s>>>(sorted, (const S*)payload, tp.T, tp.C, D,
-                                                 tp.tbits, (int)G, nparts, (S*)out_sum, omask,
-                                                 walk, tickets, tp.status, 0, (S*)out_values,
-                                                 nullptr, vsrc);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return copy_bytes(vmask, omask, (size_t)tp.n(), s);
-}
-
 template <int DT, typename U>
 hipError_t run_totals_t(const U* sorted, const void* rows, const Tape& tp, int64_t D, int64_t nout,
                         void* out, void* tail, uint8_t* flag, void* carry, uint64_t* walk,
@@ -1620,31 +1440,6 @@ bool seg_sum_merged_applies(const Tape& tp, int64_t D, int dtype, const void* pa
                             const void* out) {
   return merged_applies(tp, D * dtype_size(dtype), payload, out);
 }
-
-bool seg_sum_joint_applies(const Tape& tp, int64_t D, int dtype, const void* payload,
-                           const void* out_sum, const void* out_values) {
-  return joint_walk_applies(tp, D * dtype_size(dtype), payload, out_sum, out_values);
-}
-
-template <typename U>
-hipError_t seg_sum_joint(const U* sorted, const void* payload, int dtype, const Tape& tp,
-                         int64_t D, void* out_sum, uint8_t* omask, void* out_values,
-                         uint8_t* vmask, int32_t* vsrc, uint64_t* walk, hipStream_t s) {
-  switch (dtype) {
-    case kF32: return seg_sum_joint_t<kF32, U>(sorted, payload, tp, D, out_sum, omask, out_values, vmask, vsrc, walk, s);
-    case kF64: return seg_sum_joint_t<kF64, U>(sorted, payload, tp, D, out_sum, omask, out_values, vmask, vsrc, walk, s);
-    case kBF16: return seg_sum_joint_t<kBF16, U>(sorted, payload, tp, D, out_sum, omask, out_values, vmask, vsrc, walk, s);
-    case kF16: return seg_sum_joint_t<kF16, U>(sorted, payload, tp, D, out_sum, omask, out_values, vmask, vsrc, walk, s);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-template hipError_t seg_sum_joint<uint32_t>(const uint32_t*, const void*, int, const Tape&,
-                                            int64_t, void*, uint8_t*, void*, uint8_t*, int32_t*,
-                                            uint64_t*, hipStream_t);
-template hipError_t seg_sum_joint<uint64_t>(const uint64_t*, const void*, int, const Tape&,
-                                            int64_t, void*, uint8_t*, void*, uint8_t*, int32_t*,
-                                            uint64_t*, hipStream_t);
 
 bool seg_sum_merged_values_apply(const Tape& tp, int64_t D, int dtype, int64_t k) {
   return merged_values_apply(tp, D * dtype_size(dtype), k);

@@ -67,10 +67,14 @@ void walk_columns(int dtype, int64_t row, int ub, int* gtot, int* G, int* ncb) {
   *G = (*gtot + *ncb - 1) / *ncb;
 }
 
-// Items per part: 1024, fewer while the tape would not give every CU two blocks.
+// Items per part: 928, fewer while the tape would not give every CU two blocks.
+// A walker of 8 lanes (128-byte rows) then has 29 items, so that whole runs from
+// its first start on still fit two batches of 16 in nearly every walker: 1024
+// items (32 each) took a third batch for the one or two that hang over (sum of
+// 4.2M records, bf16 D = 64: 239 us against 232; 896 the same).
 int walk_part(int64_t nseg, int64_t L) {
   int part = kTwMaxPart;
-  while (part > kTwThreads && nseg * ((L + part - 1) / part) < 512) part /= 2;
+  for (int h = 0; h < 2 && nseg * ((L + part - 1) / part) < 512; ++h) part /= 2;
   return part;
 }
 
@@ -79,7 +83,7 @@ int64_t state_words(int64_t nseg, int64_t L, int64_t D, int dtype, int ks, int u
   walk_columns(dtype, D * dtype_size(dtype), ub, &gtot, &G, &ncb);
   const int64_t nparts = (L + walk_part(nseg, L) - 1) / walk_part(nseg, L);
   const int64_t cols = (int64_t)G * (ub / dtype_size(dtype));
-  return nseg * nparts * ncb * (ks + 1) * cols * (int64_t)(acc_bytes(dtype) / 4) + nseg * ncb;
+  return nseg * nparts * ncb * ((ks + 1) * cols * (int64_t)(acc_bytes(dtype) / 4) + 8) + nseg * ncb;
 }
 
 }  // namespace
@@ -91,10 +95,10 @@ bool walk_applies(const Tape& tp, int64_t D, int dtype, int64_t k) {
   const int64_t row = D * dtype_size(dtype);
   const int64_t kk = k > 0 ? k : 1;
   // 24-bit times and strides, a segment's rows below 2^31 bytes of its base
-  return k <= 8 && tp.T >= 1 && tp.T <= ((int64_t)1 << 23) && row < ((int64_t)1 << 24) &&
+  return k <= 8 && tp.T >= 1 && tp.T <= ((int64_t)1 << 24) && row < ((int64_t)1 << 24) &&
          tp.C * kk < ((int64_t)1 << 24) && tp.C * row * kk < ((int64_t)1 << 24) &&
          tp.T * tp.C * row * kk < ((int64_t)1 << 31) &&
-         tp.nseg() * ((2 * tp.T + kTwThreads - 1) / kTwThreads) <= INT32_MAX;
+         tp.nseg() * (2 * tp.T / (kTwMaxPart / 4) + 1) <= INT32_MAX;
 }
 
 size_t walk_words(int64_t nseg, int64_t L, int64_t D, int dtype, int64_t k) {
@@ -110,10 +114,12 @@ size_t walk_words(int64_t nseg, int64_t L, int64_t D, int dtype, int64_t k) {
 
 hipError_t tape_walk(const void* keys, bool wide, int tbits, bool same, bool fwd, const Tape& tp,
                      int64_t D, int dtype, const void* sum_in, const void* val_in, int64_t k,
-                     void* out, uint8_t* omask, uint64_t* words, hipStream_t s) {
+                     void* out, uint8_t* omask, void* val_out, uint8_t* vmask, uint64_t* words,
+                     hipStream_t s) {
   const int64_t row = D * dtype_size(dtype);
   if (!walk_applies(tp, D, dtype, k) || !tp.status) return hipErrorInvalidValue;
-  const int ub = unit_bytes(dtype, row, (uintptr_t)sum_in | (uintptr_t)val_in | (uintptr_t)out);
+  const int ub = unit_bytes(dtype, row, (uintptr_t)sum_in | (uintptr_t)val_in | (uintptr_t)out |
+                                            (uintptr_t)val_out);
   if (!ub) return hipErrorInvalidValue;
   WalkArgs a;
   a.keys = keys;
@@ -133,17 +139,24 @@ hipError_t tape_walk(const void* keys, bool wide, int tbits, bool same, bool fwd
   a.k = k > 0 ? (int)k : 1;
   a.out = out;
   a.omask = omask;
+  a.val_out = val_out;
+  a.vmask = vmask;
   a.tickets = words;
   a.words = words + a.nseg * a.ncb;
   a.err = tp.status;
-  const int ks = val_in ? walk_slots(k) : 0;
+  const int ks = val_in || val_out ? walk_slots(k) : 0;
+  hipError_t e = hipErrorInvalidValue;
   switch (dtype) {
-    case kF32: return tape_walk_f32(a, ub, ks, fwd, s);
-    case kF64: return tape_walk_f64(a, ub, ks, fwd, s);
-    case kBF16: return tape_walk_bf16(a, ub, ks, fwd, s);
-    case kF16: return tape_walk_f16(a, ub, ks, fwd, s);
-    default: return hipErrorInvalidValue;
+    case kF32: e = tape_walk_f32(a, ub, ks, fwd, s); break;
+    case kF64: e = tape_walk_f64(a, ub, ks, fwd, s); break;
+    case kBF16: e = tape_walk_bf16(a, ub, ks, fwd, s); break;
+    case kF16: e = tape_walk_f16(a, ub, ks, fwd, s); break;
+    default: break;
   }
+  // latest-1: both masks are the same bytes, and a copy in order costs less than
+  // a second byte at every random record (5 us against 13 at 4.2M records)
+  if (e == hipSuccess && val_out && k == 1) e = copy_bytes(vmask, omask, (size_t)tp.n(), s);
+  return e;
 }
 
 Tape merged_tape(const Tape& tp) {

@@ -316,7 +316,7 @@ def joint_backward_applies(T: int, C: int, D: int, k: int, element_size: int) ->
     library's own rule (its workspace query is not 0), in plain arithmetic that
     torch.compile can trace."""
     step = C * D * element_size * k  # gradient bytes of one time step
-    return (1 <= k <= 8 and 1 <= T <= 1 << 23 and C * k < 1 << 24 and step < 1 << 24
+    return (1 <= k <= 8 and 1 <= T <= 1 << 24 and C * k < 1 << 24 and step < 1 << 24
             and T * step < 1 << 31)
 
 

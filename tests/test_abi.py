@@ -254,8 +254,8 @@ def test_split_hook_and_split_workspaces():
         lib.ravel_em_latest_k_workspace(2, 64, 3, 11, 4, 0, 0, 1)
 
 
-@pytest.mark.parametrize("T,C,D,k", [(1, 1, 1, 1), (4096, 8, 64, 8), (4096, 8, 64, 9), (1 << 23, 1, 1, 1),
-                                     ((1 << 23) + 1, 1, 1, 1), (65536, 16, 128, 8), (65536, 16, 64, 8),
+@pytest.mark.parametrize("T,C,D,k", [(1, 1, 1, 1), (4096, 8, 64, 8), (4096, 8, 64, 9), (1 << 24, 1, 1, 1),
+                                     ((1 << 24) + 1, 1, 1, 1), (65536, 16, 128, 8), (65536, 16, 64, 8),
                                      (3, 1 << 20, 8, 1), (3, 1 << 19, 7, 2), (0, 3, 4, 1)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64])
 def test_joint_backward_shape_rule_matches_the_library(T, C, D, k, dtype):
