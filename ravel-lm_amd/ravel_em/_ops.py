@@ -32,6 +32,18 @@ def eager(*tensors: Optional[Tensor]) -> bool:
     return all(t is None or type(t) is torch.Tensor for t in tensors)
 
 
+# No functorch transform and no dispatch mode may watch a call that takes the
+# autograd functions at the end of this file instead of the custom ops.
+_transforms = getattr(torch._C, "_are_functorch_transforms_active", None)
+_modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
+
+
+def eager_graph(*tensors: Optional[Tensor]) -> bool:
+    """eager() for a call that records an autograd graph."""
+    return (_transforms is not None and _modes is not None and eager(*tensors)
+            and not _transforms() and _modes() == 0)
+
+
 # ------------------------------------------------------------- latest-k --
 
 
@@ -94,8 +106,7 @@ def _latest_k_fake(write_addresses, payloads, read_addresses, write_mask, addres
     )
 
 
-@torch.library.custom_op("ravel_em::latest_k_backward", mutates_args=())
-def latest_k_backward(src: Tensor, grad_values: Tensor, chain: bool) -> Tensor:
+def latest_k_backward_impl(src: Tensor, grad_values: Tensor, chain: bool) -> Tensor:
     lib = nat.library()
     B, T, C, k, D = grad_values.shape
     grad_values = grad_values.contiguous()
@@ -111,6 +122,11 @@ def latest_k_backward(src: Tensor, grad_values: Tensor, chain: bool) -> Tensor:
     if not chain:  # the sorted form's workspace carries a status word
         nat.after_call(ws)
     return grad_payload
+
+
+@torch.library.custom_op("ravel_em::latest_k_backward", mutates_args=())
+def latest_k_backward(src: Tensor, grad_values: Tensor, chain: bool) -> Tensor:
+    return latest_k_backward_impl(src, grad_values, chain)
 
 
 @latest_k_backward.register_fake
@@ -192,8 +208,7 @@ def _seg_sum_fake(write_addresses, payloads, read_addresses, write_mask, address
     return payloads.new_empty(B, T, C, D), torch.empty(B, T, C, dtype=torch.bool, device=payloads.device)
 
 
-@torch.library.custom_op("ravel_em::seg_sum_backward", mutates_args=())
-def seg_sum_backward(
+def seg_sum_backward_impl(
     write_addresses: Tensor,
     read_addresses: Optional[Tensor],
     write_mask: Optional[Tensor],
@@ -217,6 +232,18 @@ def seg_sum_backward(
     )
     nat.after_call(ws)
     return grad_payload
+
+
+@torch.library.custom_op("ravel_em::seg_sum_backward", mutates_args=())
+def seg_sum_backward(
+    write_addresses: Tensor,
+    read_addresses: Optional[Tensor],
+    write_mask: Optional[Tensor],
+    grad_sum: Tensor,
+    address_space: int,
+) -> Tensor:
+    return seg_sum_backward_impl(write_addresses, read_addresses, write_mask, grad_sum,
+                                 address_space)
 
 
 @seg_sum_backward.register_fake
@@ -320,8 +347,7 @@ def joint_backward_applies(T: int, C: int, D: int, k: int, element_size: int) ->
             and T * step < 1 << 31)
 
 
-@torch.library.custom_op("ravel_em::latest_k_sum_backward", mutates_args=())
-def latest_k_sum_backward(
+def latest_k_sum_backward_impl(
     write_addresses: Tensor,
     read_addresses: Optional[Tensor],
     write_mask: Optional[Tensor],
@@ -354,6 +380,21 @@ def latest_k_sum_backward(
     )
     nat.after_call(ws)
     return grad_payload
+
+
+@torch.library.custom_op("ravel_em::latest_k_sum_backward", mutates_args=())
+def latest_k_sum_backward(
+    write_addresses: Tensor,
+    read_addresses: Optional[Tensor],
+    write_mask: Optional[Tensor],
+    grad_values: Optional[Tensor],
+    grad_sum: Optional[Tensor],
+    address_space: int,
+    k: int,
+    taped: bool,
+) -> Tensor:
+    return latest_k_sum_backward_impl(write_addresses, read_addresses, write_mask, grad_values,
+                                      grad_sum, address_space, k, taped)
 
 
 @latest_k_sum_backward.register_fake
@@ -411,8 +452,7 @@ def _tape_dtype(address_space: int) -> torch.dtype:
     return torch.int32 if address_space < 1 << 32 else torch.int64
 
 
-@torch.library.custom_op("ravel_em::latest_k_taped", mutates_args=())
-def latest_k_taped(
+def latest_k_taped_impl(
     write_addresses: Tensor,
     payloads: Tensor,
     read_addresses: Optional[Tensor],
@@ -435,6 +475,19 @@ def latest_k_taped(
         nat.ptr(tape), nat.stream_of(payloads),
     )
     return values, mask, tape
+
+
+@torch.library.custom_op("ravel_em::latest_k_taped", mutates_args=())
+def latest_k_taped(
+    write_addresses: Tensor,
+    payloads: Tensor,
+    read_addresses: Optional[Tensor],
+    write_mask: Optional[Tensor],
+    address_space: int,
+    k: int,
+) -> Tuple[Tensor, Tensor, Tensor]:
+    return latest_k_taped_impl(write_addresses, payloads, read_addresses, write_mask,
+                               address_space, k)
 
 
 @latest_k_taped.register_fake
@@ -465,6 +518,97 @@ def _latest_k_taped_grad(ctx, grad_values, _grad_mask, _grad_tape):
 
 
 latest_k_taped.register_autograd(_latest_k_taped_grad, setup_context=_latest_k_taped_setup)
+
+
+# ------------------------------------------------- eager training calls --
+#
+# The same forwards and backwards as torch.autograd.Functions, for plain eager
+# calls (eager_graph()): the dispatcher and the custom ops' autograd wrapper cost
+# some 90 us of host time a training step (bf16 latest-4 of 262k records, whose
+# kernels take 46 us: 151 us a step through the ops).  Their backwards go through
+# the custom ops where a graph of the gradient itself is recorded (no op has a
+# second derivative: it raises then, as before) or the gradient is no plain tensor.
+
+
+def direct(op, impl, *grads: Optional[Tensor]):
+    """impl where a backward may call it directly, else the custom op."""
+    return impl if not torch.is_grad_enabled() and eager_graph(*grads) else op
+
+
+class LatestKFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, payloads, write_addresses, read_addresses, write_mask, address_space, k):
+        ctx.chain = read_addresses is None and write_mask is None
+        B, T, C, D = payloads.shape
+        ctx.taped = not ctx.chain and joint_backward_applies(T, C, D, k, payloads.element_size())
+        if ctx.taped:
+            values, mask, saved = latest_k_taped_impl(write_addresses, payloads, read_addresses,
+                                                      write_mask, address_space, k)
+        else:
+            values, mask, saved = latest_k_impl(write_addresses, payloads, read_addresses,
+                                                write_mask, address_space, k, True)
+        ctx.save_for_backward(saved)
+        ctx.args = (address_space, k)
+        ctx.mark_non_differentiable(mask)
+        ctx.set_materialize_grads(False)
+        return values, mask
+
+    @staticmethod
+    def backward(ctx, grad_values, _grad_mask):
+        (saved,) = ctx.saved_tensors
+        if grad_values is None:
+            return (None,) * 6
+        if ctx.taped:
+            g = direct(latest_k_sum_backward, latest_k_sum_backward_impl, grad_values)(
+                saved, None, None, grad_values, None, *ctx.args, True)
+        else:
+            g = direct(latest_k_backward, latest_k_backward_impl, grad_values)(
+                saved, grad_values, ctx.chain)
+        return g, None, None, None, None, None
+
+
+class SegSumFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, payloads, write_addresses, read_addresses, write_mask, address_space):
+        out, mask = seg_sum_impl(write_addresses, payloads, read_addresses, write_mask,
+                                 address_space)
+        ctx.save_for_backward(write_addresses, read_addresses, write_mask)
+        ctx.address_space = address_space
+        ctx.mark_non_differentiable(mask)
+        ctx.set_materialize_grads(False)
+        return out, mask
+
+    @staticmethod
+    def backward(ctx, grad_sum, _grad_mask):
+        saved = ctx.saved_tensors
+        if grad_sum is None:
+            return (None,) * 5
+        g = direct(seg_sum_backward, seg_sum_backward_impl, grad_sum)(
+            *saved, grad_sum, ctx.address_space)
+        return g, None, None, None, None
+
+
+class LatestKSumFn(torch.autograd.Function):
+    """For the shapes of joint_backward_applies()."""
+
+    @staticmethod
+    def forward(ctx, payloads, write_addresses, read_addresses, write_mask, address_space, k):
+        values, mask, _, out, smask = latest_k_sum_impl(write_addresses, payloads, read_addresses,
+                                                        write_mask, address_space, k, False)
+        ctx.save_for_backward(write_addresses, read_addresses, write_mask)
+        ctx.args = (address_space, k)
+        ctx.mark_non_differentiable(mask, smask)
+        ctx.set_materialize_grads(False)
+        return values, mask, out, smask
+
+    @staticmethod
+    def backward(ctx, grad_values, _grad_mask, grad_sum, _grad_smask):
+        saved = ctx.saved_tensors
+        if grad_values is None and grad_sum is None:
+            return (None,) * 6
+        g = direct(latest_k_sum_backward, latest_k_sum_backward_impl, grad_values, grad_sum)(
+            *saved, grad_values, grad_sum, *ctx.args, False)
+        return g, None, None, None, None, None
 
 
 # ------------------------------------------------------- direct C calls --

@@ -39,9 +39,9 @@ def _mfma_ok(payloads: Tensor, weight: Tensor) -> bool:
             and weight.shape[0] >= 1 and aligned)
 
 
-@torch.library.custom_op("ravel_em::latest1_linear", mutates_args=())
-def _latest1_linear(write_addresses: Tensor, payloads: Tensor, read_addresses: Optional[Tensor],
-                    weight: Tensor, address_space: int) -> Tuple[Tensor, Tensor]:
+def _latest1_linear_impl(write_addresses: Tensor, payloads: Tensor,
+                         read_addresses: Optional[Tensor], weight: Tensor,
+                         address_space: int) -> Tuple[Tensor, Tensor]:
     B, T, C, P = payloads.shape
     M = weight.shape[0]
     dev = payloads.device
@@ -64,6 +64,12 @@ def _latest1_linear(write_addresses: Tensor, payloads: Tensor, read_addresses: O
     return out, s.view(B, T, C)
 
 
+@torch.library.custom_op("ravel_em::latest1_linear", mutates_args=())
+def _latest1_linear(write_addresses: Tensor, payloads: Tensor, read_addresses: Optional[Tensor],
+                    weight: Tensor, address_space: int) -> Tuple[Tensor, Tensor]:
+    return _latest1_linear_impl(write_addresses, payloads, read_addresses, weight, address_space)
+
+
 @_latest1_linear.register_fake
 def _latest1_linear_fake(write_addresses, payloads, read_addresses, weight, address_space):
     B, T, C, P = payloads.shape
@@ -71,8 +77,7 @@ def _latest1_linear_fake(write_addresses, payloads, read_addresses, weight, addr
             torch.empty(B, T, C, dtype=torch.int32, device=payloads.device))
 
 
-@torch.library.custom_op("ravel_em::latest1_weight_grad", mutates_args=())
-def _weight_grad(payloads: Tensor, src: Tensor, grad2d: Tensor) -> Tensor:
+def _weight_grad_impl(payloads: Tensor, src: Tensor, grad2d: Tensor) -> Tensor:
     """grad2d^T [M, B*T] times the looked-up rows [B*T, C*P] (zeros where src < 0)."""
     B, T, C, P = payloads.shape
     M = grad2d.shape[1]
@@ -89,6 +94,11 @@ def _weight_grad(payloads: Tensor, src: Tensor, grad2d: Tensor) -> Tensor:
         return out
     rows = gather_read_rows(payloads, src)
     return torch.matmul(grad2d.t(), rows.reshape(B * T, C * P))
+
+
+@torch.library.custom_op("ravel_em::latest1_weight_grad", mutates_args=())
+def _weight_grad(payloads: Tensor, src: Tensor, grad2d: Tensor) -> Tensor:
+    return _weight_grad_impl(payloads, src, grad2d)
 
 
 @_weight_grad.register_fake
@@ -121,7 +131,7 @@ def _setup(ctx, inputs, output):
     ctx.set_materialize_grads(False)  # no zero gradient of the sources
 
 
-def _grads(ctx, grad_out, need_payload: bool, need_weight: bool):
+def _grads(ctx, grad_out, need_payload: bool, need_weight: bool, weight_grad, lookup_grad):
     """ravel_lm/triton_memory.py:428-475: grad_weight = grad^T @ read_flat,
     grad_payload = scatter of grad @ weight through the sources."""
     src, payloads, weight = ctx.saved_tensors
@@ -130,21 +140,44 @@ def _grads(ctx, grad_out, need_payload: bool, need_weight: bool):
     grad2d = grad_out.reshape(B * T, M).to(payloads.dtype)
     grad_weight = grad_payload = None
     if need_weight:
-        grad_weight = _weight_grad(payloads, src, grad2d.contiguous()).to(weight.dtype)
+        grad_weight = weight_grad(payloads, src, grad2d.contiguous()).to(weight.dtype)
     if need_payload:
         grad_read = torch.matmul(grad2d, weight).reshape(B, T, C, 1, P).contiguous()
-        grad_payload = _ops.latest_k_backward(src.view(B, T, C, 1), grad_read, ctx.chain)
+        grad_payload = lookup_grad(src.view(B, T, C, 1), grad_read, ctx.chain)
     return grad_payload, grad_weight
 
 
 def _backward(ctx, grad_out, _grad_src):
     if grad_out is None:
         return (None,) * 5
-    gp, gw = _grads(ctx, grad_out, ctx.needs_input_grad[1], ctx.needs_input_grad[3])
+    gp, gw = _grads(ctx, grad_out, ctx.needs_input_grad[1], ctx.needs_input_grad[3],
+                    _weight_grad, _ops.latest_k_backward)
     return None, gp, None, gw, None
 
 
 _latest1_linear.register_autograd(_backward, setup_context=_setup)
+
+
+class _Latest1LinearFn(torch.autograd.Function):
+    """The op for plain eager training calls (see _ops, eager training calls)."""
+
+    @staticmethod
+    def forward(ctx, write_addresses, payloads, read_addresses, weight, address_space):
+        out, src = _latest1_linear_impl(write_addresses, payloads, read_addresses, weight,
+                                        address_space)
+        ctx.save_for_backward(src, payloads, weight)
+        ctx.chain = read_addresses is None
+        ctx.set_materialize_grads(False)
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        if grad_out is None:
+            return (None,) * 5
+        gp, gw = _grads(ctx, grad_out, ctx.needs_input_grad[1], ctx.needs_input_grad[3],
+                        _ops.direct(_weight_grad, _weight_grad_impl, grad_out),
+                        _ops.direct(_ops.latest_k_backward, _ops.latest_k_backward_impl, grad_out))
+        return None, gp, None, gw, None
 
 
 @torch.library.custom_op("ravel_em::latest1_linear_gen", mutates_args=())
@@ -200,7 +233,8 @@ def _setup_gen(ctx, inputs, output):
 def _backward_gen(ctx, grad_out, _grad_src):
     if grad_out is None:
         return (None,) * 13
-    gp, gw = _grads(ctx, grad_out, ctx.needs_input_grad[4], ctx.needs_input_grad[5])
+    gp, gw = _grads(ctx, grad_out, ctx.needs_input_grad[4], ctx.needs_input_grad[5],
+                    _weight_grad, _ops.latest_k_backward)
     return (None, None, None, None, gp, gw) + (None,) * 7
 
 
@@ -255,8 +289,10 @@ def fused_latest1_linear(
 
     key_dtype = _composite_key_dtype(B, T, C, address_space)
     w, r = _prepare(write_addresses, read_addresses, key_dtype)
-    out, _ = _latest1_linear(w, payloads.contiguous(), r, weight.to(payloads.dtype).contiguous(),
-                             int(address_space))
+    p, wt = payloads.contiguous(), weight.to(payloads.dtype).contiguous()
+    if _ops.eager_graph(w, p, r, wt):
+        return _Latest1LinearFn.apply(w, p, r, wt, int(address_space))
+    out, _ = _latest1_linear(w, p, r, wt, int(address_space))
     return out
 
 

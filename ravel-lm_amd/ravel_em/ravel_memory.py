@@ -132,6 +132,8 @@ def causal_last_k_lookup(
     m = None if write_mask is None else write_mask.bool().contiguous()
     want_src = torch.is_grad_enabled() and payloads.requires_grad
     p = payloads.contiguous()
+    if want_src and _ops.eager_graph(w, p, r, m):
+        return _ops.LatestKFn.apply(p, w, r, m, int(address_space), int(k))
     if want_src and (r is not None or m is not None) and _ops.joint_backward_applies(
             T, C, p.shape[-1], int(k), p.element_size()):
         values, mask, _ = _ops.latest_k_taped(w, p, r, m, int(address_space), int(k))
@@ -219,6 +221,8 @@ def causal_sum_lookup(
     m = None if write_mask is None else write_mask.bool().contiguous()
     p = payloads.contiguous()
     graph = torch.is_grad_enabled() and p.requires_grad
+    if graph and _ops.eager_graph(w, p, r, m):
+        return _ops.SegSumFn.apply(p, w, r, m, int(address_space))
     op = _ops.seg_sum_impl if not graph and _ops.eager(w, p, r, m) else _ops.seg_sum
     return op(w, p, r, m, int(address_space))
 
@@ -274,6 +278,8 @@ def causal_last_k_and_sum_lookup(
     # the sources are kept only for the shapes whose backward needs them
     want_src = graph and not _ops.joint_backward_applies(T, C, p.shape[-1], int(k),
                                                          p.element_size())
+    if graph and not want_src and _ops.eager_graph(w, p, r, m):
+        return _ops.LatestKSumFn.apply(p, w, r, m, int(address_space), int(k))
     values, mask, _, summed, sum_mask = op(w, p, r, m, int(address_space), int(k), want_src)
     return values, mask, summed, sum_mask
 

@@ -235,3 +235,46 @@ def test_joint_gradient(device, case):
         if which == (0, 1):
             bits = {2: torch.int16, 4: torch.int32, 8: torch.int64}[got.element_size()]
             assert torch.equal(got.view(bits), run(0, 1).view(bits)), "two runs differ"
+
+
+@pytest.mark.parametrize("sep,masked", [(False, False), (True, False), (False, True)])
+def test_eager_functions_equal_the_custom_ops(device, sep, masked):
+    """Plain eager training calls take autograd functions: same results and
+    gradients as the custom ops bit for bit, saved tensors go through the hooks,
+    a missing gradient is none, and a second derivative raises as the ops do."""
+    from ravel_em import _ops, causal_last_k_and_sum_lookup
+
+    B, T, C, D, A, k = 2, 300, 3, 16, 11, 3
+    g = torch.Generator().manual_seed(5)
+    w = torch.randint(0, A, (B, T, C), generator=g, dtype=torch.int32).to(device)
+    r = torch.randint(0, A, (B, T, C), generator=g, dtype=torch.int32).to(device) if sep else None
+    m = (torch.rand(B, T, generator=g) < 0.6).to(device) if masked else None
+    p = torch.randn(B, T, C, D, generator=g).to(device).requires_grad_(True)
+    gv = torch.randn(B, T, C, k, D, generator=g).to(device)
+    gs = torch.randn(B, T, C, D, generator=g).to(device)
+    kw = dict(address_space=A, write_mask=m)
+    pairs = [
+        (lambda: causal_last_k_lookup(w, p, r, k=k, **kw)[:1],
+         lambda: _ops.latest_k(w, p, r, m, A, k, True)[:1] if r is None and m is None
+         else _ops.latest_k_taped(w, p, r, m, A, k)[:1], (gv,)),
+        (lambda: causal_sum_lookup(w, p, r, **kw)[:1],
+         lambda: _ops.seg_sum(w, p, r, m, A)[:1], (gs,)),
+        (lambda: causal_last_k_and_sum_lookup(w, p, r, k=k, **kw)[0::2],
+         lambda: _ops.latest_k_sum(w, p, r, m, A, k, False)[0::3], (gv, gs)),
+    ]
+    for fn, op, grads in pairs:
+        a, b = fn(), op()
+        ga, = torch.autograd.grad(a, p, grads, retain_graph=True)
+        gb, = torch.autograd.grad(b, p, grads)
+        assert all(torch.equal(x, y) for x, y in zip(a, b)) and torch.equal(ga, gb)
+        seen = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(t), t.clone())[1],
+                                                      lambda t: t):
+            c = fn()
+        gc, = torch.autograd.grad(c, p, grads)
+        assert seen and torch.equal(gc, ga)
+        lead = [x.clone().requires_grad_(True) for x in grads]
+        gg, = torch.autograd.grad(a, p, lead, create_graph=True)
+        with pytest.raises(RuntimeError):
+            gg.sum().backward()
+        assert torch.autograd.grad(a[0], p, grads[0], allow_unused=True)[0] is not None
