@@ -77,7 +77,7 @@ struct WalkArgs {
   int same;              // items are records, else reads and writes
   int tbits;             // bits of the item index in a key
   int64_t nseg, T, L, C;
-  int part;              // items per part (232, 464 or 928)
+  int part;              // items per part (at most 928)
   int64_t nparts;
   int G, gtot, ncb;      // lanes per walker, units per row, column blocks
   const void* sum_in;    // rows [B,T,C,D] or null
