@@ -1213,9 +1213,18 @@ __global__ __launch_bounds__(kMergedThreads) __attribute__((amdgpu_waves_per_eu(
   }
 }
 
+// One block a segment leaves CUs idle where segments are few, and its time grows
+// with the segment: there the sort and the segmented walk of many parts are
+// faster (bf16 D = 64, T = 4096, separate reads, 8 / 64 / 128 / 192 segments: sum
+// 49 / 57 / 64 / 69 us here against 35 / 45 / 61 / 75; joint k = 4 81 / 84 / 146 /
+// 169 against 38 / 68 / 100 / 135; T = 2048, 64: 38 against 30; T = 1024, 64: 21
+// against 25).  The rule does not look at k: the joint call's sums are those of
+// the sum alone, bit for bit.
+bool few_long_segments(const Tape& tp) { return tp.nseg() <= 112 && tp.T >= 1536; }
+
 bool merged_applies(const Tape& tp, int64_t row_bytes, const void* payload, const void* out) {
   const int64_t G = row_bytes / 16;
-  return tp.mode == kWrap && tp.T >= 1 && 2 * tp.T <= kMergedItems &&
+  return tp.mode == kWrap && !few_long_segments(tp) && tp.T >= 1 && 2 * tp.T <= kMergedItems &&
          tp.abits + tp.tbits + 1 <= 32 &&
          row_bytes % 16 == 0 && G >= 1 && G <= 64 && (G & (G - 1)) == 0 &&
          (((uintptr_t)payload | (uintptr_t)out) & 15) == 0 && tp.nseg() <= INT32_MAX &&

@@ -332,3 +332,19 @@ def test_sum_wide_rows_backward(device, shape, dtype, D):
     # fixed order, so the chain is bounded by n only.
     depth = sum_depth(T, D, dtype) if r is None and m is None else T
     compare_sums(grad.cpu(), want, scale, n, dtype, depth, f"wide backward {shape} {dtype}")
+
+
+@pytest.mark.parametrize("B,C,T", [(14, 8, 1535), (14, 8, 1536), (113, 1, 1536), (1, 1, 4096),
+                                   (15, 8, 1600)])
+@pytest.mark.parametrize("sep,masked", [(False, False), (True, False), (True, True)])
+def test_sum_on_both_sides_of_the_few_segments_rule(device, B, C, T, sep, masked):
+    """112 segments of 1536 records and longer are sorted and walked in parts,
+    more or shorter ones take one block each."""
+    A, D = 90, 16
+    g = torch.Generator().manual_seed(B + T)
+    w = torch.randint(0, A, (B, T, C), generator=g)
+    r = torch.randint(0, A, (B, T, C), generator=g) if sep else None
+    m = (torch.rand(B, T, generator=g) < 0.6) if masked else None
+    p = torch.randn(B, T, C, D, generator=g).to(torch.bfloat16)
+    check_sum(w.to(device), p.to(device), None if r is None else r.to(device), A=A,
+              mask=None if m is None else m.to(device))
