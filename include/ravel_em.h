@@ -41,7 +41,10 @@ enum {
   RAVEL_EM_INT32 = 1,
   RAVEL_EM_INT64 = 2,
   RAVEL_EM_ADDR_GEN = 3, /* address code only: addresses produced from a ravel_em_addr_gen */
-  RAVEL_EM_TAPE = 6,     /* address code of ravel_em_latest_k_sum_bwd only: a ravel_em_tape() */
+  /* address codes of ravel_em_latest_k_sum_bwd only: */
+  RAVEL_EM_TAPE = 6,      /* a ravel_em_tape() */
+  RAVEL_EM_KEYS = 7,      /* kept sorted keys of a tape with reads or a mask of its own */
+  RAVEL_EM_KEYS_SAME = 8, /* kept sorted keys of a tape whose reads are its writes */
   RAVEL_EM_FLOAT32 = 10,
   RAVEL_EM_BFLOAT16 = 11,
   RAVEL_EM_FLOAT16 = 12,
@@ -386,6 +389,31 @@ int ravel_em_seg_sum_bwd(const void* write_addr, const void* read_addr, int addr
  * what a caller keeps between the two passes when the addresses themselves may
  * change.
  */
+/*
+ * The forward sum, and the joint forward, of a training step that keeps the
+ * sorted keys they make for their backward: ravel_em_seg_sum_fwd and
+ * ravel_em_latest_k_sum_fwd with out_keys (ravel_em_tape_keys_bytes() bytes, 16-byte
+ * aligned; k = 1 for the sum).  The backward takes the keys in place of the
+ * addresses and the mask (addr_dtype RAVEL_EM_KEYS, or RAVEL_EM_KEYS_SAME when the
+ * forward had neither reads nor a mask; write_addr the keys, read_addr and
+ * write_mask NULL, the same B, T, C, A) and does not sort.  A query of 0: the
+ * forward of this shape sorts nothing that a backward could use (RAVEL_EM_EINVAL
+ * from the keeping calls).
+ */
+size_t ravel_em_tape_keys_bytes(int64_t B, int64_t T, int64_t C, int64_t D, int64_t A, int64_t k,
+                                int has_read, int has_mask, int payload_dtype);
+int ravel_em_seg_sum_fwd_keep(const void* write_addr, const void* read_addr, int addr_dtype,
+                              const uint8_t* write_mask, const void* payload, int payload_dtype,
+                              int64_t B, int64_t T, int64_t C, int64_t D, int64_t A, void* out_sum,
+                              uint8_t* out_mask, void* out_keys, size_t keys_bytes,
+                              void* workspace, size_t workspace_bytes, void* stream);
+int ravel_em_latest_k_sum_fwd_keep(const void* write_addr, const void* read_addr, int addr_dtype,
+                                   const uint8_t* write_mask, const void* payload,
+                                   int payload_dtype, int64_t B, int64_t T, int64_t C, int64_t D,
+                                   int64_t A, int64_t k, void* out_values, uint8_t* out_mask,
+                                   void* out_sum, uint8_t* out_sum_mask, void* out_keys,
+                                   size_t keys_bytes, void* workspace, size_t workspace_bytes,
+                                   void* stream);
 size_t ravel_em_tape_bytes(int64_t B, int64_t T, int64_t C, int64_t A);
 int ravel_em_tape(const void* write_addr, const void* read_addr, int addr_dtype,
                   const uint8_t* write_mask, int64_t B, int64_t T, int64_t C, int64_t A,

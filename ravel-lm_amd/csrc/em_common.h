@@ -223,6 +223,8 @@ hipError_t sort_tape(const AddrIn& addr, const uint8_t* wmask, const Tape& tp,
                      U* ka, U* kb, uint32_t* counts, U** sorted, hipStream_t s,
                      uint32_t* zero = nullptr, int64_t zero_words = 0,
                      int32_t* link_seg = nullptr);
+// Whether sort_tape (without link_seg) leaves the sorted keys in kb.
+bool sort_ends_in_b(const Tape& tp, size_t key_bytes);
 size_t sort_counts_words(const Tape& tp);
 size_t sort_fused_words(const Tape& tp, size_t key_bytes);
 

@@ -1534,6 +1534,13 @@ hipError_t sort_tape(const AddrIn& addr, const uint8_t* wmask, const Tape& tp, U
   return hipSuccess;
 }
 
+bool sort_ends_in_b(const Tape& tp, size_t key_bytes) {
+  const int npass = (tp.abits + 7) / 8;
+  if (key_bytes == 4 && tp.fused && sort_short_applies(tp, false)) return false;
+  if (tp.fused && fused_plan(tp, key_bytes).TT) return npass <= 1 || npass % 2 == 1;
+  return npass % 2 == 1;
+}
+
 template <typename U>
 hipError_t emit_order(const U* sorted, const uint8_t* wmask, int64_t* vprefix, const Tape& tp,
                       void* out_keys, bool keys64, int64_t* out_order, hipStream_t s, int64_t b0,

@@ -18,7 +18,8 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
 # dtype codes (include/ravel_em.h)
 INT32, INT64 = 1, 2
 ADDR_GEN = 3  # address code: write/read pointers are AddrGen descriptors
-TAPE = 6  # address code of the joint backward: write pointer is a merged tape
+# address codes of the joint backward: the write pointer is a merged tape, or kept sorted keys
+TAPE, KEYS, KEYS_SAME = 6, 7, 8
 FLOAT32, BFLOAT16, FLOAT16, FLOAT64 = 10, 11, 12, 13
 
 _PAYLOAD_CODES = {
@@ -100,6 +101,16 @@ SIGNATURES = {
     "ravel_em_seg_sum_bwd_workspace": (_sz, [_i64, _i64, _i64, _i64, _i64, _i, _i, _i]),
     "ravel_em_seg_sum_bwd": (
         _i, [_vp, _vp, _i, _vp, _vp, _i, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _sz, _vp]
+    ),
+    "ravel_em_tape_keys_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64, _i64, _i, _i, _i]),
+    "ravel_em_seg_sum_fwd_keep": (
+        _i, [_vp, _vp, _i, _vp, _vp, _i, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _sz, _vp, _sz,
+             _vp]
+    ),
+    "ravel_em_latest_k_sum_fwd_keep": (
+        _i,
+        [_vp, _vp, _i, _vp, _vp, _i, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp,
+         _sz, _vp, _sz, _vp],
     ),
     "ravel_em_tape_bytes": (_sz, [_i64, _i64, _i64, _i64]),
     "ravel_em_tape": (_i, [_vp, _vp, _i, _vp, _i64, _i64, _i64, _i64, _vp, _vp]),

@@ -167,8 +167,10 @@ def seg_sum_impl(
     read_addresses: Optional[Tensor],
     write_mask: Optional[Tensor],
     address_space: int,
+    keys: Optional[Tensor] = None,
 ) -> Tuple[Tensor, Tensor]:
-    """The body of ravel_em::seg_sum (also called directly, see eager)."""
+    """The body of ravel_em::seg_sum (also called directly, see eager); the
+    sorted keys of the tape go to `keys` when given (kept_keys)."""
     lib = nat.library()
     B, T, C = write_addresses.shape
     D = payloads.shape[-1]
@@ -180,11 +182,12 @@ def seg_sum_impl(
         B, T, C, D, address_space, int(read_addresses is not None), int(write_mask is not None), code
     )
     ws = nat.workspace(nbytes, dev)
+    keep = () if keys is None else (nat.ptr(keys), keys.numel())
     _call(
-        lib.ravel_em_seg_sum_fwd,
+        lib.ravel_em_seg_sum_fwd if keys is None else lib.ravel_em_seg_sum_fwd_keep,
         nat.ptr(write_addresses), nat.ptr(read_addresses), nat.addr_code(write_addresses.dtype),
         nat.ptr(write_mask), nat.ptr(payloads), code, B, T, C, D, address_space,
-        nat.ptr(out), nat.ptr(mask), nat.ptr(ws), ws.numel(), nat.stream_of(payloads),
+        nat.ptr(out), nat.ptr(mask), *keep, nat.ptr(ws), ws.numel(), nat.stream_of(payloads),
     )
     nat.after_call(ws)
     return out, mask
@@ -281,9 +284,11 @@ def latest_k_sum_impl(
     address_space: int,
     k: int,
     want_src: bool,
+    keys: Optional[Tensor] = None,
 ) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
     """The body of ravel_em::latest_k_sum (also called directly, see eager):
-    (values, mask, src, sum, sum_mask) of one tape in one C call."""
+    (values, mask, src, sum, sum_mask) of one tape in one C call; the sorted keys
+    of the tape go to `keys` when given (kept_keys; then no sources)."""
     lib = nat.library()
     B, T, C = write_addresses.shape
     D = payloads.shape[-1]
@@ -298,13 +303,16 @@ def latest_k_sum_impl(
         B, T, C, D, address_space, k, int(read_addresses is not None), int(write_mask is not None),
         int(want_src), code)
     ws = nat.workspace(nbytes, dev)
-    _call(
-        lib.ravel_em_latest_k_sum_fwd,
-        nat.ptr(write_addresses), nat.ptr(read_addresses), nat.addr_code(write_addresses.dtype),
-        nat.ptr(write_mask), nat.ptr(payloads), code, B, T, C, D, address_space, k,
-        nat.ptr(values), nat.ptr(mask), nat.ptr(src) if want_src else None, nat.ptr(out),
-        nat.ptr(smask), nat.ptr(ws), ws.numel(), nat.stream_of(payloads),
-    )
+    tape = (nat.ptr(write_addresses), nat.ptr(read_addresses), nat.addr_code(write_addresses.dtype),
+            nat.ptr(write_mask), nat.ptr(payloads), code, B, T, C, D, address_space, k,
+            nat.ptr(values), nat.ptr(mask))
+    work = (nat.ptr(ws), ws.numel(), nat.stream_of(payloads))
+    if keys is None:
+        _call(lib.ravel_em_latest_k_sum_fwd, *tape, nat.ptr(src) if want_src else None,
+              nat.ptr(out), nat.ptr(smask), *work)
+    else:
+        _call(lib.ravel_em_latest_k_sum_fwd_keep, *tape, nat.ptr(out), nat.ptr(smask),
+              nat.ptr(keys), keys.numel(), *work)
     nat.after_call(ws)
     return values, mask, src, out, smask
 
@@ -356,10 +364,12 @@ def latest_k_sum_backward_impl(
     address_space: int,
     k: int,
     taped: bool,
+    keys: int = 0,
 ) -> Tensor:
     """Payload gradient of latest_k (grad_values [B,T,C,k,D]), of seg_sum
     (grad_sum [B,T,C,D]) or of both of one tape; with ``taped`` the first
-    argument is the tape that latest_k_taped returned."""
+    argument is the tape that latest_k_taped returned, with `keys` (nat.KEYS or
+    nat.KEYS_SAME) the sorted keys that the forward kept."""
     lib = nat.library()
     gv = None if grad_values is None else grad_values.contiguous()
     gs = None if grad_sum is None else grad_sum.contiguous()
@@ -368,13 +378,14 @@ def latest_k_sum_backward_impl(
     grad_payload = g.new_empty(B, T, C, D)
     code = nat.payload_code(g.dtype)
     nbytes = lib.ravel_em_latest_k_sum_bwd_workspace(
-        B, T, C, D, address_space, k, int(taped or read_addresses is not None),
+        B, T, C, D, address_space, k,
+        int(taped or keys == nat.KEYS or read_addresses is not None),
         int(write_mask is not None), code)
     ws = nat.workspace(nbytes, g.device)
     _call(
         lib.ravel_em_latest_k_sum_bwd,
         nat.ptr(write_addresses), nat.ptr(read_addresses),
-        nat.TAPE if taped else nat.addr_code(write_addresses.dtype), nat.ptr(write_mask),
+        keys or (nat.TAPE if taped else nat.addr_code(write_addresses.dtype)), nat.ptr(write_mask),
         nat.ptr(gv), nat.ptr(gs), code, B, T, C, D, address_space, k, nat.ptr(grad_payload),
         nat.ptr(ws), ws.numel(), nat.stream_of(g),
     )
@@ -567,12 +578,24 @@ class LatestKFn(torch.autograd.Function):
         return g, None, None, None, None, None
 
 
+def kept_keys(payloads, read_addresses, write_mask, address_space, k) -> Optional[Tensor]:
+    """Room for the sorted keys that a training forward keeps for its backward
+    (None where the forward of the shape sorts nothing that the backward uses):
+    4 or 8 bytes a record, twice that with separate reads or a mask."""
+    B, T, C, D = payloads.shape
+    n = nat.library().ravel_em_tape_keys_bytes(
+        B, T, C, D, address_space, k, int(read_addresses is not None), int(write_mask is not None),
+        nat.payload_code(payloads.dtype))
+    return torch.empty(n, dtype=torch.uint8, device=payloads.device) if n else None
+
+
 class SegSumFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, payloads, write_addresses, read_addresses, write_mask, address_space):
+        keys = kept_keys(payloads, read_addresses, write_mask, address_space, 1)
         out, mask = seg_sum_impl(write_addresses, payloads, read_addresses, write_mask,
-                                 address_space)
-        ctx.save_for_backward(write_addresses, read_addresses, write_mask)
+                                 address_space, keys)
+        ctx.save_for_backward(write_addresses, read_addresses, write_mask, keys)
         ctx.address_space = address_space
         ctx.mark_non_differentiable(mask)
         ctx.set_materialize_grads(False)
@@ -580,12 +603,20 @@ class SegSumFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_sum, _grad_mask):
-        saved = ctx.saved_tensors
+        *tape, keys = ctx.saved_tensors
         if grad_sum is None:
             return (None,) * 5
-        g = direct(seg_sum_backward, seg_sum_backward_impl, grad_sum)(
-            *saved, grad_sum, ctx.address_space)
+        fn = direct(seg_sum_backward, seg_sum_backward_impl, grad_sum)
+        if keys is not None and fn is seg_sum_backward_impl:
+            g = latest_k_sum_backward_impl(keys, None, None, None, grad_sum, ctx.address_space, 1,
+                                           False, _keys_code(tape))
+        else:
+            g = fn(*tape, grad_sum, ctx.address_space)
         return g, None, None, None, None
+
+
+def _keys_code(tape) -> int:
+    return nat.KEYS_SAME if tape[1] is None and tape[2] is None else nat.KEYS
 
 
 class LatestKSumFn(torch.autograd.Function):
@@ -593,9 +624,10 @@ class LatestKSumFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, payloads, write_addresses, read_addresses, write_mask, address_space, k):
+        keys = kept_keys(payloads, read_addresses, write_mask, address_space, k)
         values, mask, _, out, smask = latest_k_sum_impl(write_addresses, payloads, read_addresses,
-                                                        write_mask, address_space, k, False)
-        ctx.save_for_backward(write_addresses, read_addresses, write_mask)
+                                                        write_mask, address_space, k, False, keys)
+        ctx.save_for_backward(write_addresses, read_addresses, write_mask, keys)
         ctx.args = (address_space, k)
         ctx.mark_non_differentiable(mask, smask)
         ctx.set_materialize_grads(False)
@@ -603,11 +635,14 @@ class LatestKSumFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_values, _grad_mask, grad_sum, _grad_smask):
-        saved = ctx.saved_tensors
+        *tape, keys = ctx.saved_tensors
         if grad_values is None and grad_sum is None:
             return (None,) * 6
-        g = direct(latest_k_sum_backward, latest_k_sum_backward_impl, grad_values, grad_sum)(
-            *saved, grad_values, grad_sum, *ctx.args, False)
+        fn = direct(latest_k_sum_backward, latest_k_sum_backward_impl, grad_values, grad_sum)
+        if keys is not None and fn is latest_k_sum_backward_impl:
+            g = fn(keys, None, None, grad_values, grad_sum, *ctx.args, False, _keys_code(tape))
+        else:
+            g = fn(*tape, grad_values, grad_sum, *ctx.args, False)
         return g, None, None, None, None, None
 
 

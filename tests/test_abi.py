@@ -267,3 +267,23 @@ def test_joint_backward_shape_rule_matches_the_library(T, C, D, k, dtype):
                                                           nat.payload_code(dtype))
     want = _ops.joint_backward_applies(T, C, D, k, torch.empty(0, dtype=dtype).element_size())
     assert (n > 0) == (want or T == 0)
+
+
+def test_keeping_calls_check_their_keys_without_a_device():
+    """The room for sorted keys: none where one block a segment sums without a
+    sort; the size and alignment are refused before any HIP call."""
+    lib = nat.library()
+    shape = (2, 5000, 3, 16, 200)
+    n = lib.ravel_em_tape_keys_bytes(*shape, 1, 0, 0, nat.BFLOAT16)
+    assert n == 2 * 5000 * 3 * 4
+    assert lib.ravel_em_tape_keys_bytes(*shape, 1, 1, 0, nat.BFLOAT16) == 2 * n
+    assert lib.ravel_em_tape_keys_bytes(2, 300, 3, 16, 200, 1, 0, 0, nat.BFLOAT16) == 0
+    assert lib.ravel_em_tape_keys_bytes(*shape, 9, 0, 0, nat.BFLOAT16) == 0
+    fake = ctypes.c_void_p(0x1000)  # never dereferenced: the checks come first
+    for keys, size, rc in ((fake, n - 1, 3), (ctypes.c_void_p(0x1008), n, 1), (None, n, 1)):
+        assert rc == lib.ravel_em_seg_sum_fwd_keep(
+            fake, None, nat.INT64, None, fake, nat.BFLOAT16, *shape, fake, fake, keys, size, fake,
+            1 << 30, None)
+        assert rc == lib.ravel_em_latest_k_sum_fwd_keep(
+            fake, None, nat.INT64, None, fake, nat.BFLOAT16, *shape, 1, fake, fake, fake, fake,
+            keys, size, fake, 1 << 30, None)

@@ -278,3 +278,32 @@ def test_eager_functions_equal_the_custom_ops(device, sep, masked):
         with pytest.raises(RuntimeError):
             gg.sum().backward()
         assert torch.autograd.grad(a[0], p, grads[0], allow_unused=True)[0] is not None
+
+
+@pytest.mark.parametrize("sep,masked", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("B,T,C,A", [(2, 5000, 3, 200), (1, 4200, 2, 70000), (1, 4300, 1, 1 << 21),
+                                     (2, 2000, 2, 30)])
+def test_kept_keys_give_the_gradient_of_the_sorted_addresses(device, sep, masked, B, T, C, A):
+    """A training forward that sorts keeps its keys: the backward that walks them
+    equals, bit for bit, the one that sorts the addresses again (keys of one to
+    three digit passes, 32 and 64 bits, and a tape sorted by one block a segment)."""
+    from ravel_em import _ops, causal_last_k_and_sum_lookup
+
+    D, k = 16, 2
+    g = torch.Generator().manual_seed(T)
+    w = torch.randint(0, A, (B, T, C), generator=g).to(device)
+    r = torch.randint(0, A, (B, T, C), generator=g).to(device) if sep else None
+    m = (torch.rand(B, T, generator=g) < 0.7).to(device) if masked else None
+    p = torch.randn(B, T, C, D, generator=g).to(torch.bfloat16).to(device).requires_grad_(True)
+    gv = torch.randn(B, T, C, k, D, generator=g).to(torch.bfloat16).to(device)
+    gs = torch.randn(B, T, C, D, generator=g).to(torch.bfloat16).to(device)
+    keys = _ops.kept_keys(p, r, m, A, k)
+    records = B * T * C * (2 if sep or masked else 1)
+    assert keys.numel() in (4 * records, 8 * records)
+    summed = causal_sum_lookup(w, p, r, address_space=A, write_mask=m)[0]
+    got, = torch.autograd.grad(summed, p, gs)
+    assert torch.equal(summed, _ops.seg_sum(w, p, r, m, A)[0])
+    assert torch.equal(got, _ops.seg_sum_backward(w, r, m, gs, A))
+    vals, _, summed, _ = causal_last_k_and_sum_lookup(w, p, r, address_space=A, k=k, write_mask=m)
+    got, = torch.autograd.grad((vals, summed), p, (gv, gs))
+    assert torch.equal(got, _ops.latest_k_sum_backward(w, r, m, gv, gs, A, k, False))
